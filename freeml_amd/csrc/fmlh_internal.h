@@ -149,6 +149,9 @@ struct GemmArgs {
     const float* R = nullptr;
     int ldr = 0;
     KvDest kv;  // kEpiKV only
+    // Rows to plan the product for instead of M (0: M): parts of one product then take the same
+    // tiles and K ranges, so that a row's result does not depend on how many parts there are.
+    int plan_rows = 0;
     // ln_g != nullptr: A holds rows before a LayerNorm (LayerNormOp, eps ln_eps, gamma ln_g,
     // optional beta ln_b) and the product takes the normalised rows.  Skinny NT products only
     // (gemm_takes_ln); no normalised copy is written.
@@ -158,22 +161,24 @@ struct GemmArgs {
     hipStream_t s = nullptr;
 };
 
-// Kernel choice for a shape: skinny kernels for M <= 8 (decode), MFMA tiles otherwise, with
-// the split-K factor and the workspace (floats) the split partial sums need.
+// Kernel choice for a shape: skinny kernels for M <= 8 (decode), fp32 MFMA tiles for the batched
+// decode's rows, split bf16 tiles (gemm_split.hip) above, with the split-K factor and the
+// workspace (floats) the partial sums need.
 struct GemmPlan {
-    enum Kind { kSkinnyNN, kSkinnyNT, kMfma, kMfmaNT } kind = kMfma;
+    enum Kind { kSkinnyNN, kSkinnyNT, kMfma, kSplit } kind = kMfma;
     int bm = 64, bn = 64;
     int splits = 1, k_per_split = 0;
     size_t ws_elems = 0;
 };
-GemmPlan plan_gemm(int M, int N, int K, int b_trans);
+// one_range: without splitting K (kEpiKV writes its results as they are).
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false);
 
 // Runs the product.  ws/ws_elems: caller workspace for split partials (must hold
 // plan_gemm(...).ws_elems floats); nullptr uses a process-wide buffer grown on demand, which
 // callers that capture HIP graphs must avoid.
 int gemm(const GemmArgs& g, float* ws, size_t ws_elems);
-// Whether the product runs on gemm_nt_kernel (the kernel that takes kEpiKV): B stored N x K,
-// 16-byte aligned K-contiguous rows, K % 16 == 0 and enough 64 x 64 tiles.
+// Whether the product runs on the split bf16 tiles with B stored N x K (they take kEpiKV):
+// 16-byte aligned K-contiguous rows and K % 16 == 0.
 bool gemm_runs_nt(const GemmArgs& g);
 // Whether the product can take its A rows through a LayerNorm (GemmArgs ln_*): the skinny NT
 // kernels (M <= 8, B stored N x K) with K <= 1024.
@@ -182,7 +187,7 @@ bool gemm_takes_ln(int M, int N, int K, int b_trans);
 // *splits partial M x N sums, [split][row][col], for a caller-side reduction (fused with what
 // follows the product).  Otherwise launches nothing and sets *splits = 0.
 int gemm_split_partials(const GemmArgs& g, float* ws, size_t ws_elems, int* splits);
-// The K-split partial sums of an NT product (B stored N x K) on gemm_nt_kernel's 64 x 64 tiles,
+// The K-split partial sums of an NT product (B stored N x K) on 64 x 64 split bf16 tiles,
 // whatever the plan: split z takes K range [z K / splits, (z + 1) K / splits) and writes
 // ws[z][M][N], for a caller-side reduction.  K must be a multiple of 16 splits.
 int gemm_nt_partials(const GemmArgs& g, int splits, float* ws, size_t ws_elems);

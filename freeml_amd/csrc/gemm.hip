@@ -1,12 +1,11 @@
 // GEMM kernels behind Mul / MatMul_Strided and the token loop's projections.
 //
-//  * gemm_nt_kernel: fp32 MFMA (v_mfma_f32_32x32x2f32) tiles for B stored N x K (the token
-//    loop's weights), operands copied straight into a three-stage LDS ring; used when the
-//    product has at least half a device's worth of 64 x 64 tiles (prefill).
-//  * gemm_mfma_kernel: the same MFMA tiling with register-staged, double-buffered LDS, for
-//    either B layout and M > 8 (batched decode, small products).  Optional split-K writes
-//    partial sums that splitk_reduce_kernel adds in a fixed order (deterministic) before the
-//    epilogue.
+//  * gemm_split_kernel (gemm_split.hip): everything wider than the batched decode, each fp32
+//    operand split into three bf16 parts on the bf16 matrix cores.
+//  * gemm_mfma_kernel: fp32 MFMA tiles (v_mfma_f32_32x32x2f32) with register-staged,
+//    double-buffered LDS, for either B layout and 8 < M <= 64 (batched decode).  Optional
+//    split-K writes partial sums that splitk_reduce_kernel adds in a fixed order
+//    (deterministic) before the epilogue.
 //  * skinny kernels for M <= 8 (single-sequence decode): HBM-bound weight streaming, every
 //    weight read once, all M rows accumulated per weight load.
 //  * gemm_strided_kernel: any transpose mode and element strides (MatMul_Strided views).
@@ -15,6 +14,7 @@
 // sequentially over k; these kernels sum in other orders, so results differ from it by fp32
 // rounding only (compared with a tolerance in the parity tests).
 #include "fmlh_internal.h"
+#include "gemm_split.h"
 
 #include <algorithm>
 #include <cstdio>
@@ -221,258 +221,19 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ partial, int spli
 }
 
 // ---------------------------------------------------------------------------------------
-// NT tile kernel (B stored N x K: the projections' transposed weights).  Both operands are
-// K-contiguous, so a KBT-wide K block of either tile is R rows of KBT/4 float4, which the wave
-// copies from global memory straight into LDS (global_load_lds, 16 bytes per lane, 1 KB per
-// instruction: 16 rows of a 16-wide block, 8 rows of a 32-wide one) without passing through
-// registers.  Three LDS stages: the copies of block k+2 are in flight while block k is
-// multiplied, with one barrier per block.  The 64 x 64 tiles take 32-wide blocks: 16 MFMAs per
-// wave between barriers (measured on MI355X at the prefill projection shapes, 3 work-groups per
-// CU: 10-15 % faster than 16-wide blocks at 6 per CU, whose waves wait at a barrier every 8).
-// A copy instruction fills 1 KB of LDS contiguously, so rows cannot be padded; instead float4
-// q of row r is stored at position q ^ nt_swz(r), which puts the operand reads of any 8 or 16
-// consecutive lanes (one row each, same q) on distinct banks.  Rows past M (columns past N)
-// copy row M-1 (N-1): their results are computed and never stored.  Same MFMA operand layout
-// as gemm_mfma_kernel; lane half h takes the block's k = h KBT/2 .. + KBT/2 - 1.
-// ---------------------------------------------------------------------------------------
-// Depends on r % 16 only.  4 quads per row: ((r >> 1) ^ (r >> 3)) & 3; 8 quads per row:
-// (r >> 1) & 7 with bit 2 flipped on odd rows (8 consecutive rows: 0 4 1 5 2 6 3 7).
-__device__ __forceinline__ int quad_swz(int r) { return ((r >> 1) ^ ((r >> 3) & 1)) & 3; }
-template <int KBT>
-__device__ __forceinline__ int nt_swz(int r) {
-    if constexpr (KBT == 16) return quad_swz(r);
-    else return ((r >> 1) & 7) ^ ((r & 1) << 2);
-}
-
-constexpr int NT_STAGES = 3;
-constexpr int NT_KB64 = 32;  // K block of the 64 x 64 tiles
-
-// Whether the 64 x 64 NT tiles take 32-wide K blocks for a K range of k (FMLH_GEMM_NT_KB=16:
-// 16-wide blocks everywhere, for comparison).
-bool nt_wide_kb(int k) {
-    static const bool narrow = [] {
-        const char* e = std::getenv("FMLH_GEMM_NT_KB");
-        return e && std::strcmp(e, "16") == 0;
-    }();
-    return !narrow && k % NT_KB64 == 0;
-}
-
-template <int BM, int BN, int KBT = KB>
-constexpr size_t nt_lds_bytes() { return (size_t)NT_STAGES * (BM + BN) * KBT * sizeof(float); }
-
-// SPLIT: work-group z of the grid's third dimension takes K range [z K, z K + K) (K is the
-// range length) and writes its partial sums to partial[z][M][N] (epilogue by the reduction).
-// K must be a multiple of KBT.
-template <int BM, int BN, int EPI, bool SPLIT = false, int KBT = KB>
-__global__ __launch_bounds__(256) void gemm_nt_kernel(
-    const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
-    float* C, int ldc, int M, int N, int K, const float* R, int ldr, KvDest kv,
-    float* __restrict__ partial = nullptr) {
-    static_assert(!SPLIT || EPI == kEpiNone, "split partials take no epilogue");
-    static_assert(BM % 64 == 0 && BN % 64 == 0, "tile must be a multiple of 64");
-    static_assert(KBT == 16 || KBT == 32, "K block of 16 or 32");
-    constexpr int WM = BM / 2, WN = BN / 2;
-    constexpr int MB = WM / 32, NB = WN / 32;
-    constexpr int A_FL = BM * KBT, ST_FL = (BM + BN) * KBT;
-    constexpr int QPR = KBT / 4, RPI = 64 / QPR;   // float4 per row, rows per copy instruction
-    constexpr int NQ = QPR / 2;                    // float4 operand reads per row and block
-    constexpr int DA = BM / (4 * RPI), DB = BN / (4 * RPI);  // copy instructions per wave per block
-    constexpr int D = DA + DB;
-
-    extern __shared__ __attribute__((aligned(16))) float nt_lds[];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int h = lane >> 5, c = lane & 31;
-    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
-    const int nk = K / KBT;
-
-    // Copy addressing: lane -> row (lane / QPR) of an RPI-row chunk and stored position
-    // lane % QPR, which holds global float4 (lane % QPR) ^ nt_swz(row).
-    const int crow = lane / QPR, cpos = lane % QPR;
-    const int cq = cpos ^ nt_swz<KBT>(crow);  // chunks start at multiples of 8 rows: r % 16 ...
-    const int cq8 = cpos ^ nt_swz<KBT>(crow + 8);  // ... is crow or crow + 8
-    const float* asrc[DA];
-    const float* bsrc[DB];
-    const size_t kofs = SPLIT ? (size_t)blockIdx.z * K : 0;
-#pragma unroll
-    for (int t = 0; t < DA; ++t) {
-        const int r = RPI * (wave + 4 * t);
-        const int gr = min(row0 + r + crow, M - 1);
-        asrc[t] = A + (size_t)gr * lda + kofs + 4 * ((r & 8) ? cq8 : cq);
-    }
-#pragma unroll
-    for (int t = 0; t < DB; ++t) {
-        const int r = RPI * (wave + 4 * t);
-        const int gc = min(col0 + r + crow, N - 1);
-        bsrc[t] = B + (size_t)gc * ldb + kofs + 4 * ((r & 8) ? cq8 : cq);
-    }
-    auto issue = [&](int kb, int st) {
-        float* sa = nt_lds + st * ST_FL;
-        float* sb = sa + A_FL;
-#pragma unroll
-        for (int t = 0; t < DA; ++t) copy16_to_lds(sa + (wave + 4 * t) * 256, asrc[t] + kb * KBT);
-#pragma unroll
-        for (int t = 0; t < DB; ++t) copy16_to_lds(sb + (wave + 4 * t) * 256, bsrc[t] + kb * KBT);
-    };
-
-    // Operand reads: lane (h, c) takes float4 h NQ .. h NQ + NQ - 1 of its row
-    // (k = h KBT/2 .. h KBT/2 + KBT/2 - 1); rows wm WM + 32 i + c have r % 16 = c % 16.
-    const int swc = nt_swz<KBT>(c);
-
-    floatx16 acc[MB][NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    issue(0, 0);
-    if (nk > 1) issue(1, 1);
-    int st = 0;
-    for (int kb = 0; kb < nk; ++kb) {
-        // This wave's copies of block kb are done once at most those of block kb+1 remain;
-        // the barrier makes every wave's part visible and ends all reads of the stage that
-        // block kb+2 overwrites (it held block kb-1).
-        // (__syncthreads would wait for every copy in flight, block kb+1's included.)
-        if (kb + 1 < nk) copies_barrier<D>();
-        else copies_barrier<0>();
-        if (kb + 2 < nk) issue(kb + 2, st == 0 ? 2 : st - 1);
-        const float* sa = nt_lds + st * ST_FL;
-        const float* sb = sa + A_FL;
-        floatx4 av[NQ][MB], bv[NQ][NB];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int pos = (h * NQ + q) ^ swc;
-#pragma unroll
-            for (int i = 0; i < MB; ++i)
-                av[q][i] = *reinterpret_cast<const floatx4*>(sa + (wm * WM + 32 * i + c) * KBT + 4 * pos);
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-                bv[q][j] = *reinterpret_cast<const floatx4*>(sb + (wn * WN + 32 * j + c) * KBT + 4 * pos);
-        }
-#pragma unroll
-        for (int s = 0; s < 4 * NQ; ++s) {
-#pragma unroll
-            for (int i = 0; i < MB; ++i) {
-#pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s / 4][i][s % 4], bv[s / 4][j][s % 4],
-                                                                     acc[i][j], 0, 0, 0);
-            }
-        }
-        // All operand reads first (first quads first: the first MFMAs wait for those only),
-        // then the MFMAs, which the later reads overlap.
-        __builtin_amdgcn_sched_group_barrier(0x100, NQ * (MB + NB), 0);  // LDS reads
-        __builtin_amdgcn_sched_group_barrier(0x008, 4 * NQ * MB * NB, 0);  // MFMA
-        st = st == NT_STAGES - 1 ? 0 : st + 1;
-    }
-
-    // kEpiKV: cache offset of each row of the tile, (sequence * H * T + position) * head_dim.
-    __shared__ size_t kv_row[EPI == kEpiKV ? BM : 1];
-    int kv_shift = 0;
-    if constexpr (EPI == kEpiKV) {
-        kv_shift = 31 - __builtin_clz(kv.hd);
-        for (int rr = tid; rr < BM; rr += 256) {
-            const int gr = min(row0 + rr, M - 1);
-            const int b = gr / kv.rows_per_seq, p = gr - b * kv.rows_per_seq;
-            kv_row[rr] = ((size_t)b * kv.H * kv.T + p) << kv_shift;
-        }
-        __syncthreads();
-    }
-    if constexpr (BM == 64 && BN == 64) {
-        // The tile goes through LDS (the operand ring is free once every wave is past the
-        // barrier below: every copy has landed and every read of the ring is done), then out
-        // as 16-byte stores of whole row segments (a key/value tile row is one head's cache
-        // row for head_dim 64, or 2-4 of them), where the destination's strides and alignment
-        // allow it; otherwise the per-element stores below.
-        const bool rows_ok = ((uintptr_t)C % 16 == 0) && ldc % 4 == 0 &&
-                             (EPI != kEpiResid || ((uintptr_t)R % 16 == 0 && ldr % 4 == 0));
-        const bool vec_ok = SPLIT ? (N % 4 == 0 && (uintptr_t)partial % 16 == 0)
-                                  : (EPI == kEpiKV || (N % 4 == 0 && rows_ok));
-        if (vec_ok) {
-            constexpr int TS = BN + 4;  // padded row: the 16-byte reads stay aligned
-            float* tile = nt_lds;
-            if constexpr (EPI != kEpiKV) __syncthreads();  // (kEpiKV passed one above)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                tile[(wm * 32 + 8 * (r / 4) + 4 * h + (r % 4)) * TS + wn * 32 + c] = acc[0][0][r];
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < BM * BN / 4 / 256; ++u) {
-                const int idx = tid + 256 * u, rr = idx / (BN / 4), q = idx % (BN / 4);
-                const int gr = row0 + rr, gc = col0 + 4 * q;
-                if (gr >= M || gc >= N) continue;  // N % 4 == 0: no float4 crosses N
-                floatx4 v = *reinterpret_cast<const floatx4*>(tile + rr * TS + 4 * q);
-                if constexpr (SPLIT) {
-                    *reinterpret_cast<floatx4*>(partial + ((size_t)blockIdx.z * M + gr) * N + gc) = v;
-                } else if constexpr (EPI == kEpiKV) {
-                    if (gc < kv.C) {
-                        *reinterpret_cast<floatx4*>(C + (size_t)gr * ldc + gc) = v;
-                    } else {
-                        const bool is_v = gc >= 2 * kv.C;
-                        const int cc = gc - (is_v ? 2 * kv.C : kv.C);
-                        const int hh = cc >> kv_shift, d = cc & (kv.hd - 1);
-                        float* cache = is_v ? kv.vc : kv.kc;
-                        *reinterpret_cast<floatx4*>(cache + kv_row[rr] + ((size_t)hh * kv.T << kv_shift) + d) = v;
-                    }
-                } else {
-                    if constexpr (EPI == kEpiResid) {
-                        const floatx4 rv = *reinterpret_cast<const floatx4*>(R + (size_t)gr * ldr + gc);
-                        v += rv;
-                    } else if constexpr (EPI != kEpiNone) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = epilogue<EPI>(v[e], R, 0);
-                    }
-                    *reinterpret_cast<floatx4*>(C + (size_t)gr * ldc + gc) = v;
-                }
-            }
-            return;
-        }
-    }
-
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int gc = col0 + wn * WN + j * 32 + c;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int gr = row0 + wm * WM + i * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-                if (gr < M && gc < N) {
-                    if constexpr (SPLIT) {
-                        partial[((size_t)blockIdx.z * M + gr) * N + gc] = acc[i][j][r];
-                    } else if constexpr (EPI == kEpiKV) {
-                        if (gc < kv.C) {
-                            C[(size_t)gr * ldc + gc] = acc[i][j][r];
-                        } else {
-                            // head_dim is a power of two; the row's cache offset comes from LDS
-                            const bool is_v = gc >= 2 * kv.C;
-                            const int cc = gc - (is_v ? 2 * kv.C : kv.C);
-                            const int hh = cc >> kv_shift, d = cc & (kv.hd - 1);
-                            float* cache = is_v ? kv.vc : kv.kc;
-                            cache[kv_row[gr - row0] + ((size_t)hh * kv.T << kv_shift) + d] = acc[i][j][r];
-                        }
-                    } else {
-                        C[(size_t)gr * ldc + gc] = epilogue<EPI>(acc[i][j][r], R, (size_t)gr * ldr + gc);
-                    }
-                }
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------
 // Split-K NT kernel for short K ranges (batched decode: M <= 64 rows, K-range of at most
 // kNtSplitMaxBlocks 16-wide blocks per work-group).  The whole range of both 64 x 64 tiles is
 // copied into LDS at once (one stage per block), so the work-group waits for global memory
 // once instead of once per block; then every MFMA runs back to back.  Writes the partial sums
-// of split blockIdx.z to partial[z][M][N] (added up by the caller).  Same operand layout, LDS
-// swizzle and k order as gemm_nt_kernel.
+// of split blockIdx.z to partial[z][M][N] (added up by the caller).  Same operand layout and
+// k order as gemm_mfma_kernel.
 // ---------------------------------------------------------------------------------------
 constexpr int kNtSplitMaxBlocks = 8;
+
+// Float4 q of a 16-float row r is stored at q ^ quad_swz(r), which puts the operand reads of any 8
+// or 16 consecutive lanes (one row each, same q) on distinct banks (a direct-to-LDS copy fills
+// LDS contiguously, so rows cannot be padded).
+__device__ __forceinline__ int quad_swz(int r) { return ((r >> 1) ^ ((r >> 3) & 1)) & 3; }
 
 __global__ __launch_bounds__(256) void gemm_nt_split_kernel(
     const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, int M, int N,
@@ -1038,51 +799,21 @@ int mfma_tile(const GemmArgs& g, int splits, int kps, float* ws) {
                      : mfma_epi<BM, BN, false>(g, splits, kps, ws);
 }
 
-template <int BM, int BN, int EPI>
-int launch_nt_tile(const GemmArgs& g) {
-    dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM);
-    if (BM == 64 && BN == 64 && nt_wide_kb(g.K)) {
-        const size_t lds = nt_lds_bytes<BM, BN, NT_KB64>();
-        hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, EPI, false, NT_KB64>), grid, dim3(256), lds, g.s,
-                           g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, g.K, g.R, g.ldr, g.kv);
-    } else {
-        const size_t lds = nt_lds_bytes<BM, BN>();
-        hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, EPI>), grid, dim3(256), lds, g.s,
-                           g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, g.K, g.R, g.ldr, g.kv);
-    }
-    FMLH_LAUNCHED("gemm_nt_kernel");
-    return FMLH_OK;
+SplitGemm split_args(const GemmArgs& g, int tile) {
+    SplitGemm q;
+    q.A = g.A; q.lda = g.lda; q.B = g.B; q.ldb = g.ldb; q.b_kc = g.b_trans != 0;
+    q.C = g.C; q.ldc = g.ldc; q.M = g.M; q.N = g.N; q.K = g.K; q.epi = g.epi; q.R = g.R; q.ldr = g.ldr;
+    q.kv = g.kv; q.tile = tile; q.s = g.s;
+    return q;
 }
 
-// 64 x 64 NT partial sums over `splits` K ranges of k_per_split (multiple of KB) each.
-void launch_nt_partials(const GemmArgs& g, int splits, int k_per_split, float* ws) {
-    dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, splits);
-    if (nt_wide_kb(k_per_split)) {
-        const size_t lds = nt_lds_bytes<64, 64, NT_KB64>();
-        hipLaunchKernelGGL((gemm_nt_kernel<64, 64, kEpiNone, true, NT_KB64>), grid, dim3(256), lds, g.s,
-                           g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, k_per_split, g.R, g.ldr, g.kv, ws);
-    } else {
-        const size_t lds = nt_lds_bytes<64, 64>();
-        hipLaunchKernelGGL((gemm_nt_kernel<64, 64, kEpiNone, true>), grid, dim3(256), lds, g.s,
-                           g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, k_per_split, g.R, g.ldr, g.kv, ws);
-    }
-}
-
-// NT tiles with split K (plan splits > 1): partials, then the reduction with the epilogue.
-int launch_nt_split_tiles(const GemmArgs& g, const GemmPlan& p, float* ws) {
-    launch_nt_partials(g, p.splits, p.k_per_split, ws);
-    FMLH_LAUNCHED("gemm_nt_kernel(split)");
+// A planned split product: one launch, or K ranges and their reduction with the epilogue.
+int run_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
+    SplitGemm q = split_args(g, p.bm);
+    if (p.splits == 1) return gemm_split(q);
+    q.epi = kEpiNone; q.splits = p.splits; q.k_per_split = p.k_per_split; q.partial = ws;
+    FMLH_TRY(gemm_split(q));
     return reduce_dispatch(g.epi, ws, p.splits, g.C, g.ldc, g.M, g.N, g.R, g.ldr, g.s);
-}
-
-template <int BM, int BN>
-int nt_epi(const GemmArgs& g) {
-    switch (g.epi) {
-        case kEpiGelu: return launch_nt_tile<BM, BN, kEpiGelu>(g);
-        case kEpiResid: return launch_nt_tile<BM, BN, kEpiResid>(g);
-        case kEpiKV: return launch_nt_tile<BM, BN, kEpiKV>(g);
-        default: return launch_nt_tile<BM, BN, kEpiNone>(g);
-    }
 }
 
 template <int EPI>
@@ -1149,7 +880,7 @@ int launch_nt_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
 
 }  // namespace
 
-GemmPlan plan_gemm(int M, int N, int K, int b_trans) {
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
     GemmPlan p;
     if (M <= SK_MAXM) {
         if (b_trans) {
@@ -1162,35 +893,43 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans) {
         return p;
     }
     const int cus = cu_count() > 0 ? cu_count() : 256;
-    // FMLH_GEMM_NT: "0" puts B-transposed products on gemm_mfma_kernel, "1" on the NT kernel
-    // whatever the tile count (for measurement).
-    const char* nt_env = std::getenv("FMLH_GEMM_NT");
-    const bool nt_forced = nt_env && nt_env[0] == '1';
-    if (b_trans && (nt_forced || (long)((M + 63) / 64) * ((N + 63) / 64) * 2 >= cus) &&
-        !(nt_env && nt_env[0] == '0')) {
-        // NT kernel, 64 x 64 tiles: measured on MI355X at the prefill projection shapes
-        // (M 4096-14336, N 384-3072, K 384-3072) within 2% of the best of 64x64, 128x64 and
-        // 128x128 everywhere (six work-groups per CU hide the operand-read latency, and small
-        // tiles leave no CU idle at the end).  FMLH_GEMM_NT_TILE=128x128|128x64 selects the others.
-        p.kind = GemmPlan::kMfmaNT;
-        p.bm = 64;
-        p.bn = 64;
-        // Fewer than two 64 x 64 tiles per CU leaves CUs idle in the last round; with a long K
-        // range, two K halves balance the grid (partials + a reduction kernel).
-        // FMLH_GEMM_NT_SPLIT_K=0 turns it off.
-        const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
-        const char* sk = std::getenv("FMLH_GEMM_NT_SPLIT_K");
-        if (!(sk && sk[0] == '0') && tiles < 2L * cus && K >= 1024 && (K / 2) % KB == 0) {
-            p.splits = 2;
-            p.k_per_split = K / 2;
-            p.ws_elems = (size_t)2 * M * N;
-        }
+    const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+    // Split bf16 tiles for everything wider than the batched decode, but for a few N x K products
+    // whose short K ranges gemm_nt_split_kernel holds in LDS at once (256 x 384 x 384: 8.2 us
+    // against 9.1; from 37 tiles or K > 768 on it is behind: 256 x 1152 x 384 11.4 against 10.5).
+    if ((M > 64 && !(b_trans && tiles64 <= 36 && K <= 768)) || (b_trans && 2 * tiles64 >= cus)) {
+        p.kind = GemmPlan::kSplit;
+        // Tile and K ranges by the time (us) they take on MI355X: a CU multiplies a 128 x 128 x 16
+        // block in 0.64 us whether it holds one work-group or three, a 64 x 64 x 32 one in 0.58
+        // alone and 0.45 among several; K ranges write and read their partials at 4 TB/s, and a
+        // reduction takes 3.5 us and 0.35 per range.
+        float best = INFINITY;
+        for (int tile : {128, 64})
+            for (int sp = 1; sp <= 8; ++sp) {
+                const size_t ws = (size_t)sp * M * N;
+                if (sp > 1 && (one_range || K / sp < 64 || ws > kNoAllocScratchFloats)) break;
+                const float units = (float)(tile == 128 ? tiles128 : tiles64) * sp / cus, kr = (float)K / sp;
+                const float t = (tile == 128 ? std::max(1.0f, units) * kr / 16 * 0.64f
+                                             : std::max(0.58f, 0.45f * units) * kr / 32) +
+                                (sp > 1 ? 3.5f + 0.35f * sp + 2e-6f * ws : 1e-6f * M * N);
+                if (t < best) {
+                    best = t;
+                    p.bm = p.bn = tile;
+                    p.splits = sp;
+                }
+            }
+        // FMLH_GEMM_NT_TILE=128x128 | 64x64 forces the tile, FMLH_GEMM_NT_SPLIT_K=n the K ranges
+        // (0: one).
         if (const char* e = std::getenv("FMLH_GEMM_NT_TILE")) {
             int bm = 0, bn = 0;
-            if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 &&
-                ((bm == 128 && (bn == 128 || bn == 64)) || (bm == 64 && bn == 64))) {
-                p.bm = bm; p.bn = bn;
-            }
+            if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 && (bm == 128 || bm == 64)) p.bm = p.bn = bm;
+        }
+        if (const char* e = one_range ? nullptr : std::getenv("FMLH_GEMM_NT_SPLIT_K")) p.splits = std::max(1, std::atoi(e));
+        if (p.splits > 1) {
+            p.k_per_split = ((K + p.splits - 1) / p.splits + 15) / 16 * 16;
+            p.splits = (K + p.k_per_split - 1) / p.k_per_split;
+            p.ws_elems = p.splits > 1 ? (size_t)p.splits * M * N : 0;
         }
         return p;
     }
@@ -1210,6 +949,15 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans) {
     return p;
 }
 
+namespace {
+// The plan of a call: that of plan_rows rows where given, with room for the call's own.
+GemmPlan plan_for(const GemmArgs& g) {
+    GemmPlan p = plan_gemm(std::max(g.M, g.plan_rows), g.N, g.K, g.b_trans, g.epi == kEpiKV);
+    if (g.plan_rows > g.M && p.splits > 1) p.ws_elems = (size_t)p.splits * g.M * g.N;
+    return p;
+}
+}  // namespace
+
 bool gemm_takes_ln(int M, int N, int K, int b_trans) {
     return M > 0 && N > 0 && K <= 64 * kSkLnNE && plan_gemm(M, N, K, b_trans).kind == GemmPlan::kSkinnyNT;
 }
@@ -1217,14 +965,14 @@ bool gemm_takes_ln(int M, int N, int K, int b_trans) {
 bool gemm_runs_nt(const GemmArgs& g) {
     const bool vec_ok = aligned16(g.A) && aligned16(g.B) && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
                         g.K % KB == 0;
-    return vec_ok && g.M > 0 && g.N > 0 && plan_gemm(g.M, g.N, g.K, g.b_trans).kind == GemmPlan::kMfmaNT;
+    return vec_ok && g.M > 0 && g.N > 0 && g.b_trans && plan_for(g).kind == GemmPlan::kSplit;
 }
 
 size_t gemm_workspace_elems(const GemmArgs& g) {
     if (g.M == 0 || g.N == 0 || g.K == 0) return 0;
     const bool vec_ok = aligned16(g.A) && aligned16(g.B) && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
                         g.K % KB == 0;
-    return vec_ok ? plan_gemm(g.M, g.N, g.K, g.b_trans).ws_elems : 0;  // the strided fallback takes none
+    return vec_ok ? plan_for(g).ws_elems : 0;  // the strided fallback takes none
 }
 
 int gemm(const GemmArgs& g, float* ws, size_t ws_elems) {
@@ -1245,7 +993,7 @@ int gemm(const GemmArgs& g, float* ws, size_t ws_elems) {
         return gemm_strided(g.b_trans ? FMLH_TRANSPOSE_RIGHT : FMLH_TRANSPOSE_NONE, g.C, g.A, g.B,
                             g.M, g.N, g.K, g.lda, 1, g.ldb, 1, g.ldc, 1, 1, 0, 0, 0, g.s);
     }
-    GemmPlan p = plan_gemm(g.M, g.N, g.K, g.b_trans);
+    const GemmPlan p = plan_for(g);
     if (p.ws_elems > ws_elems) {
         if (ws != nullptr) return set_error(FMLH_E_INVALID, "gemm: workspace too small");
         FMLH_TRY(global_workspace(p.ws_elems, &ws));
@@ -1264,11 +1012,7 @@ int gemm(const GemmArgs& g, float* ws, size_t ws_elems) {
             FMLH_LAUNCHED("skinny_nn_partial_kernel");
             return reduce_dispatch(g.epi, ws, p.splits, g.C, g.ldc, g.M, g.N, g.R, g.ldr, g.s);
         }
-        case GemmPlan::kMfmaNT:
-            if (p.splits > 1 && g.epi != kEpiKV && p.bm == 64 && p.bn == 64) return launch_nt_split_tiles(g, p, ws);
-            if (p.bm == 128 && p.bn == 128) return nt_epi<128, 128>(g);
-            if (p.bm == 128) return nt_epi<128, 64>(g);
-            return nt_epi<64, 64>(g);
+        case GemmPlan::kSplit: return run_split(g, p, ws);
         default:
             if (nt_split_applies(g, p)) {
                 FMLH_TRY(launch_nt_split(g, p, ws));
@@ -1286,9 +1030,10 @@ int gemm_nt_partials(const GemmArgs& g, int splits, float* ws, size_t ws_elems) 
                  g.M, g.N, g.K, splits);
     FMLH_REQUIRE(ws != nullptr && (size_t)splits * g.M * g.N <= ws_elems, "gemm_nt_partials: workspace too small");
     if (g.M == 0 || g.N == 0) return FMLH_OK;
-    launch_nt_partials(g, splits, g.K / splits, ws);
-    FMLH_LAUNCHED("gemm_nt_kernel(partials)");
-    return FMLH_OK;
+    SplitGemm q = split_args(g, 64);
+    q.epi = kEpiNone; q.splits = splits; q.k_per_split = g.K / splits; q.partial = ws;
+    if (splits == 1) { q.C = ws; q.ldc = g.N; }
+    return gemm_split(q);
 }
 
 int gemm_split_partials(const GemmArgs& g, float* ws, size_t ws_elems, int* splits) {

@@ -1,0 +1,462 @@
+// fp32 products on the bf16 matrix cores: gemm_split_kernel.
+//
+// Every fp32 operand element is split exactly into three bf16 parts, x = x0 + x1 + x2 (each the
+// round-to-nearest bf16 of what is left, 3 x 8 significant bits = fp32's 24), and the product
+// takes the six part products whose weight is 2^-16 or more of the whole,
+//   a b ~ a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0),
+// accumulated in fp32 by the bf16 MFMAs, smallest first.  The three left out are below 2^-24 of
+// |a b| together, under the rounding of one fp32 product.
+//
+// Why: the fp32 MFMA these products ran on reaches 154 TFLOP/s at most on MI355X (100-113 of it
+// in the kernel this one replaced); bf16 runs at 16 times its nominal rate, so six part products
+// are 2.6 times as fast at the nominal peaks.  A large library bf16 product reaches 1218
+// TFLOP/s, a sixth of which is 203: the 128 x 128 tiles reach 200 at 8192^3.  Measured, before ->
+// after (us): 4096 x 3072 x 768 stored N x K 180 -> 105, stored K x N 193 -> 110; 1024 x 50304 x
+// 768 692 -> 442.  Relative error against 64 bits (2-norm, normal operands): K 384 / 768 / 3072
+// 2.9e-7 / 4.2e-7 / 8.7e-7 (fp32 MFMA: 3.5e-7 / 5.0e-7 / 9.9e-7); with the small part products
+// summed apart (LO) 1.1e-7 / 1.6e-7 / 3.4e-7.
+//
+// The operands are split while they are staged (registers -> LDS), so fp32 matrices of any
+// layout are read once and nothing is kept.  Per 128 x 128 x 16 block a work-group's matrix cores
+// need ~770 clocks, its LDS ~580 (three planes written once, read by two waves) and its
+// vector units ~500 (5.5 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
+// every plane of half as many products) and serve the products with too few large tiles.
+#include "gemm_split.h"
+
+#include <cstdlib>
+#include <cstring>
+
+namespace fmlh {
+
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float gelu_ref(float x) { return 0.5f * x * (1.0f + erff(x / 1.41421354f)); }
+
+__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{x, y}, bf16x2));
+}
+
+// Eight floats -> their three bf16 planes (one 16-byte unit each).
+__device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&p)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x = v[2 * i], y = v[2 * i + 1];
+        const uint32_t p0 = pack_bf16(x, y);
+        const float rx = x - __uint_as_float(p0 << 16), ry = y - __uint_as_float(p0 & 0xffff0000u);
+        const uint32_t p1 = pack_bf16(rx, ry);
+        const float sx = rx - __uint_as_float(p1 << 16), sy = ry - __uint_as_float(p1 & 0xffff0000u);
+        p[0][i] = p0;
+        p[1][i] = p1;
+        p[2][i] = pack_bf16(sx, sy);
+    }
+}
+
+// Rows whose largest element is below this (and not zero) do not split exactly any more: the
+// third part falls under bf16's smallest normal.
+constexpr float kSplitTiny = 0x1p-90f;
+
+// The MFMAs of the two tile sizes.  Lane l of an MT x MT product supplies row / column l % MT and
+// the 8 consecutive k of octet l / MT; accumulator register r holds row 8 (r / 4) + 4 (l / MT) +
+// r % 4 of column l % MT.
+template <int MT>
+struct Mfma;
+template <>
+struct Mfma<32> {
+    using Acc = floatx16;
+    static constexpr int kRegs = 16, kK = 16;
+    static __device__ __forceinline__ Acc bf16(bf16x8 a, bf16x8 b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Acc fp32(float a, float b, Acc c) {  // one k per lane: l / MT
+        return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct Mfma<16> {
+    using Acc = floatx4;
+    static constexpr int kRegs = 4, kK = 32;
+    static __device__ __forceinline__ Acc bf16(bf16x8 a, bf16x8 b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Acc fp32(float a, float b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+};
+
+template <int BM, int BN, int BK, int WVM, int WVN, bool AKC, bool BKC, int EPI, bool SPLIT, bool LO, int MT>
+__global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
+    const float* __restrict__ A, int lda, size_t a_plane, const float* __restrict__ B, int ldb, size_t b_plane,
+    float* C, int ldc, size_t c_plane, int M, int N, int K, const float* R, int ldr, KvDest kv,
+    float* __restrict__ partial, int k_per_split, int tiles_m, int tiles_n) {
+    constexpr int U = BK / 8;                       // 16-byte units per row and plane
+    constexpr int NT = 64 * WVM * WVN;
+    constexpr int NA = BM * U / NT, NB = BN * U / NT;  // units a thread stages per K block
+    static_assert(NA * NT == BM * U && NB * NT == BN * U, "units must divide over the threads");
+    constexpr int WM = BM / WVM, WN = BN / WVN;
+    constexpr int MB = WM / MT, NBK = WN / MT;     // MFMA tiles per wave
+    using Acc = typename Mfma<MT>::Acc;
+    constexpr int AR = Mfma<MT>::kRegs, KM = Mfma<MT>::kK;
+    constexpr int STAGE = 3 * (BM + BN) * U;        // units per LDS stage
+    extern __shared__ __attribute__((aligned(16))) uintx4 lds[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wm = wave / WVN, wn = wave % WVN;
+    const int h = lane / MT, c = lane % MT;  // this lane's k octet and row / column of an MFMA
+
+    // Tile order: consecutive work-groups go to different XCDs, so XCD x takes a contiguous
+    // eighth of the tiles, walked in groups of 8 tile rows (their A rows and the walked B
+    // columns stay in that XCD's L2).
+    const int total = tiles_m * tiles_n;
+    int t = blockIdx.x;
+    {
+        const int per = total / 8, rem = total % 8, x = t & 7, i = t >> 3;
+        t = x * per + (x < rem ? x : rem) + i;
+    }
+    const int gsz = 8 * tiles_n, grp = t / gsz, gm = min(8, tiles_m - 8 * grp);
+    const int tm = 8 * grp + (t - grp * gsz) % gm, tn = (t - grp * gsz) / gm;
+    const int row0 = tm * BM, col0 = tn * BN;
+    const int z = blockIdx.z;
+    const int kbeg = SPLIT ? z * k_per_split : 0;
+    const int kend = SPLIT ? min(K, kbeg + k_per_split) : K;
+    if constexpr (!SPLIT) {
+        A += z * a_plane;
+        B += z * b_plane;
+        C += z * c_plane;
+    }
+
+    // Staging: unit u = tid + 256 i of an operand is 8 consecutive k of one tile row.  K
+    // contiguous: two 16-byte loads; row contiguous (stored K x rows): eight 4-byte loads,
+    // consecutive lanes on consecutive rows.
+    uint32_t a_off[NA], b_off[NB];  // bytes from the tile's base
+    int a_row[NA], a_oct[NA], b_row[NB], b_oct[NB];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int u = tid + NT * i;
+        a_row[i] = AKC ? u / U : u % BM;
+        a_oct[i] = AKC ? u % U : u / BM;
+        const uint32_t r = min(a_row[i], M - 1 - row0);
+        a_off[i] = 4u * (AKC ? r * (uint32_t)lda + 8 * a_oct[i] : 8 * a_oct[i] * (uint32_t)lda + r);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int u = tid + NT * i;
+        b_row[i] = BKC ? u / U : u % BN;
+        b_oct[i] = BKC ? u % U : u / BN;
+        const uint32_t r = min(b_row[i], N - 1 - col0);
+        b_off[i] = 4u * (BKC ? r * (uint32_t)ldb + 8 * b_oct[i] : 8 * b_oct[i] * (uint32_t)ldb + r);
+    }
+    const float* a_base = A + (AKC ? (size_t)row0 * lda : (size_t)row0);
+    const float* b_base = B + (BKC ? (size_t)col0 * ldb : (size_t)col0);
+    float va[NA][8], vb[NB][8];
+    float amax[NA], bmax[NB];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) amax[i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) bmax[i] = 0.0f;
+
+    auto load_unit = [&](float (&v)[8], const float* base, uint32_t off, bool kc, int ld, int kk, bool full) {
+        const char* p = reinterpret_cast<const char*>(base) + off;
+        if (kc) {
+            if (full) {
+                const floatx4 lo = *reinterpret_cast<const floatx4*>(p);
+                const floatx4 hi = *reinterpret_cast<const floatx4*>(p + 16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = kk + e < kend ? reinterpret_cast<const float*>(p)[e] : 0.0f;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = full || kk + e < kend ? *reinterpret_cast<const float*>(p + (size_t)4 * e * ld) : 0.0f;
+        }
+    };
+    auto load = [&](int k0, bool full) {
+        const float* ab = a_base + (AKC ? (size_t)k0 : (size_t)k0 * lda);
+        const float* bb = b_base + (BKC ? (size_t)k0 : (size_t)k0 * ldb);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) load_unit(va[i], ab, a_off[i], AKC, lda, k0 + 8 * a_oct[i], full);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) load_unit(vb[i], bb, b_off[i], BKC, ldb, k0 + 8 * b_oct[i], full);
+    };
+    // Unit o of row r is stored at o ^ swz(r): any 8 consecutive lanes, reading one row each or
+    // writing, touch 8 distinct 16-byte bank groups.
+    auto swz = [](int r) { return U == 2 ? (r >> 2) & 1 : (r >> 1) & 3; };
+    auto store = [&](int st) {
+        uintx4* sa = lds + st * STAGE;
+        uintx4* sb = sa + 3 * BM * U;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            uintx4 p[3];
+            split8(va[i], p);
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) amax[i] = fmaxf(fmaxf(amax[i], fabsf(va[i][e])), fabsf(va[i][e + 1]));
+#pragma unroll
+            for (int q = 0; q < 3; ++q) sa[(q * BM + a_row[i]) * U + (a_oct[i] ^ swz(a_row[i]))] = p[q];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            uintx4 p[3];
+            split8(vb[i], p);
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) bmax[i] = fmaxf(fmaxf(bmax[i], fabsf(vb[i][e])), fabsf(vb[i][e + 1]));
+#pragma unroll
+            for (int q = 0; q < 3; ++q) sb[(q * BN + b_row[i]) * U + (b_oct[i] ^ swz(b_row[i]))] = p[q];
+        }
+    };
+
+    Acc acc[MB][NBK], low[LO ? MB : 1][LO ? NBK : 1];
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                for (int r = 0; r < AR; ++r) acc[i][j][r] = 0.0f;
+    };
+    clear();
+    if constexpr (LO) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                for (int r = 0; r < AR; ++r) low[i][j][r] = 0.0f;
+    }
+
+    // Two LDS stages, one barrier per K block: block k + 1 (in registers since the iteration
+    // before) is split and written while block k is multiplied, block k + 2 is requested.  The
+    // barrier waits for LDS only; the requested loads stay in flight across it.  Past the last
+    // whole block the loop stages that block again (never multiplied), so its body has no branch
+    // and the split's vector instructions run beside the MFMAs.
+    auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    auto multiply = [&](int st, auto stage_next) {
+        const uintx4* sa = lds + st * STAGE;
+        const uintx4* sb = sa + 3 * BM * U;
+#pragma unroll
+        for (int ks = 0; ks < BK / KM; ++ks) {
+            const int o = KM / 8 * ks + h;
+            bf16x8 a[3][MB], b[3][NBK];
+#pragma unroll
+            for (int q = 2; q >= 0; --q) {
+#pragma unroll
+                for (int i = 0; i < MB; ++i) {
+                    const int r = wm * WM + MT * i + c;
+                    a[q][i] = __builtin_bit_cast(bf16x8, sa[(q * BM + r) * U + (o ^ swz(r))]);
+                }
+#pragma unroll
+                for (int j = 0; j < NBK; ++j) {
+                    const int r = wn * WN + MT * j + c;
+                    b[2 - q][j] = __builtin_bit_cast(bf16x8, sb[((2 - q) * BN + r) * U + (o ^ swz(r))]);
+                }
+            }
+            if (ks == 0) stage_next();
+            constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NBK; ++j) {
+                        Acc& d = LO && q < 5 ? low[LO ? i : 0][LO ? j : 0] : acc[i][j];
+                        d = Mfma<MT>::bf16(a[pa[q]][i], b[pb[q]][j], d);
+                    }
+        }
+    };
+    const int nk = (kend - kbeg) / BK;
+    if (nk > 0) {
+        load(kbeg, true);
+        store(0);
+        load(kbeg + (nk > 1 ? BK : 0), true);
+        barrier();
+        for (int kb = 0; kb < nk; ++kb) {
+            multiply(kb & 1, [&]() {
+                store((kb + 1) & 1);
+                load(kbeg + min(kb + 2, nk - 1) * BK, true);
+            });
+            barrier();
+        }
+    }
+    if (kbeg + nk * BK < kend) {  // the rest of K
+        load(kbeg + nk * BK, false);
+        store(0);
+        barrier();
+        multiply(0, []() {});
+        barrier();
+    }
+    if constexpr (LO) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NBK; ++j) acc[i][j] += low[i][j];
+    }
+    // What the split cannot carry -- infinities (and values that round to one in bf16), which
+    // leave a NaN in the sums, and rows of tiny elements -- is multiplied again in fp32.
+    {
+        uint32_t* rmax = reinterpret_cast<uint32_t*>(lds);  // free since the last barrier
+        for (int i = tid; i < BM + BN; i += NT) rmax[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NA; ++i) atomicMax(&rmax[a_row[i]], __float_as_uint(amax[i]));
+#pragma unroll
+        for (int i = 0; i < NB; ++i) atomicMax(&rmax[BM + b_row[i]], __float_as_uint(bmax[i]));
+        __syncthreads();
+        bool redo = false;
+        for (int i = tid; i < BM + BN; i += NT) {
+            const float v = __uint_as_float(rmax[i]);
+            redo |= v > 0.0f && v < kSplitTiny;
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                for (int r = 0; r < AR; ++r) redo |= acc[i][j][r] != acc[i][j][r];
+        if (__syncthreads_or(redo)) {
+            clear();
+            for (int k = kbeg; k < kend; k += 64 / MT) {
+                const int kk = min(k + h, kend - 1);
+                const bool in = k + h < kend;
+                float av[MB], bv[NBK];
+#pragma unroll
+                for (int i = 0; i < MB; ++i) {
+                    const size_t r = min(row0 + wm * WM + MT * i + c, M - 1);
+                    av[i] = in ? A[AKC ? r * lda + kk : (size_t)kk * lda + r] : 0.0f;
+                }
+#pragma unroll
+                for (int j = 0; j < NBK; ++j) {
+                    const size_t r = min(col0 + wn * WN + MT * j + c, N - 1);
+                    bv[j] = in ? B[BKC ? r * ldb + kk : (size_t)kk * ldb + r] : 0.0f;
+                }
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NBK; ++j)
+                        acc[i][j] = Mfma<MT>::fp32(av[i], bv[j], acc[i][j]);
+            }
+        }
+    }
+
+    // kEpiKV: cache offset of each row of the tile, (sequence * H * T + position) * head_dim.
+    __shared__ size_t kv_row[EPI == kEpiKV ? BM : 1];
+    if constexpr (EPI == kEpiKV) {
+        for (int rr = tid; rr < BM; rr += NT) {
+            const int gr = min(row0 + rr, M - 1);
+            const int sb = gr / kv.rows_per_seq, p = gr - sb * kv.rows_per_seq;
+            kv_row[rr] = ((size_t)sb * kv.H * kv.T + p) * kv.hd;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < NBK; ++j) {
+        const int gc = col0 + wn * WN + MT * j + c;
+        if (gc >= N) continue;
+        float* cache = nullptr;  // kEpiKV: this column's place in the K / V caches, row 0
+        if constexpr (EPI == kEpiKV) {
+            if (gc >= kv.C) {
+                const bool is_v = gc >= 2 * kv.C;
+                const int cc = gc - (is_v ? 2 * kv.C : kv.C), hh = cc / kv.hd, d = cc - hh * kv.hd;
+                cache = (is_v ? kv.vc : kv.kc) + (size_t)hh * kv.T * kv.hd + d;
+            }
+        }
+        // The residual of all the lane's rows first: C may be R, so the compiler cannot move a
+        // load above an earlier store itself (one round trip per row otherwise).
+        float res[EPI == kEpiResid ? MB : 1][EPI == kEpiResid ? AR : 1];
+        if constexpr (EPI == kEpiResid) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int r = 0; r < AR; ++r) {
+                    const int gr = min(row0 + wm * WM + MT * i + 8 * (r / 4) + 4 * h + (r % 4), M - 1);
+                    res[i][r] = R[(size_t)gr * ldr + gc];
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int r = 0; r < AR; ++r) {
+                const int lr = wm * WM + MT * i + 8 * (r / 4) + 4 * h + (r % 4), gr = row0 + lr;
+                if (gr >= M) continue;
+                const float v = acc[i][j][r];
+                if constexpr (SPLIT) {
+                    partial[((size_t)z * M + gr) * N + gc] = v;
+                } else if constexpr (EPI == kEpiKV) {
+                    if (cache) cache[kv_row[lr]] = v;
+                    else C[(size_t)gr * ldc + gc] = v;
+                } else if constexpr (EPI == kEpiGelu) {
+                    C[(size_t)gr * ldc + gc] = gelu_ref(v);
+                } else if constexpr (EPI == kEpiResid) {
+                    C[(size_t)gr * ldc + gc] = res[i][r] + v;
+                } else {
+                    C[(size_t)gr * ldc + gc] = v;
+                }
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int BK, bool AKC, bool BKC, int EPI, bool SPLIT, bool LO>
+int launch(const SplitGemm& g) {
+    const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
+    constexpr size_t lds = (size_t)2 * 3 * (BM + BN) * BK * sizeof(uint16_t);  // 48 KB
+    hipLaunchKernelGGL((gemm_split_kernel<BM, BN, BK, 2, 2, AKC, BKC, EPI, SPLIT, LO, BM == 128 ? 32 : 16>),
+                       dim3((unsigned)tm * tn, 1, SPLIT ? g.splits : g.planes), dim3(256), lds, g.s, g.A, g.lda,
+                       g.a_plane, g.B, g.ldb, g.b_plane, g.C, g.ldc, g.c_plane, g.M, g.N, g.K, g.R, g.ldr, g.kv,
+                       g.partial, g.k_per_split, tm, tn);
+    FMLH_LAUNCHED("gemm_split_kernel");
+    return FMLH_OK;
+}
+
+template <int BM, int BN, int BK, bool AKC, bool BKC>
+int by_epilogue(const SplitGemm& g) {
+    constexpr bool LO = BM == 64;  // 64 x 64 tiles have the registers for it at no cost
+    if constexpr (AKC) {
+        if (LO || !g.low) {
+            if (g.splits > 1) return launch<BM, BN, BK, AKC, BKC, kEpiNone, true, LO>(g);
+            switch (g.epi) {
+                case kEpiGelu: return launch<BM, BN, BK, AKC, BKC, kEpiGelu, false, LO>(g);
+                case kEpiResid: return launch<BM, BN, BK, AKC, BKC, kEpiResid, false, LO>(g);
+                case kEpiKV:
+                    if constexpr (BKC) return launch<BM, BN, BK, AKC, BKC, kEpiKV, false, LO>(g);
+                    break;
+                default: return launch<BM, BN, BK, AKC, BKC, kEpiNone, false, LO>(g);
+            }
+        }
+    }
+    FMLH_REQUIRE(g.epi == kEpiNone && g.splits == 1, "gemm_split: epilogue %d, %d splits of this layout", g.epi, g.splits);
+    return launch<BM, BN, BK, AKC, BKC, kEpiNone, false, true>(g);
+}
+
+template <int BM, int BN, int BK>
+int by_layout(const SplitGemm& g) {
+    if (g.a_kc) return g.b_kc ? by_epilogue<BM, BN, BK, true, true>(g) : by_epilogue<BM, BN, BK, true, false>(g);
+    return g.b_kc ? by_epilogue<BM, BN, BK, false, true>(g) : by_epilogue<BM, BN, BK, false, false>(g);
+}
+
+}  // namespace
+
+bool gemm_split_takes(const SplitGemm& g) {
+    // K-contiguous operands are read 16 bytes at a time; a tile's rows (or a K block's) must lie
+    // within 32-bit byte offsets of its first element.
+    auto vec = [](const float* p, int ld, size_t plane) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0 && plane % 4 == 0; };
+    if (g.a_kc && !vec(g.A, g.lda, g.a_plane)) return false;
+    if (g.b_kc && !vec(g.B, g.ldb, g.b_plane)) return false;
+    return g.M > 0 && g.N > 0 && g.K > 0 && g.lda < (1 << 22) && g.ldb < (1 << 22) && g.planes <= 65535;
+}
+
+int gemm_split(const SplitGemm& g) {
+    FMLH_REQUIRE(gemm_split_takes(g), "gemm_split: %dx%dx%d operands not aligned", g.M, g.N, g.K);
+    FMLH_REQUIRE(g.splits == 1 || (g.partial && g.k_per_split % 16 == 0), "gemm_split: split K without room");
+    return g.tile == 128 ? by_layout<128, 128, 16>(g) : by_layout<64, 64, 32>(g);
+}
+
+}  // namespace fmlh

@@ -794,15 +794,15 @@ int run_blocks_decode_fused(fmlh_nanollm* m, int batch) {
 // Whether a prefill of M rows runs its residual projections as two K halves whose reduction
 // adds the residual and applies the next LayerNorm (reduce_resid_ln_kernel: no LayerNorm
 // launches, and the attention projection's grid no longer leaves CUs idle).  Only where that
-// grid has fewer than two 64 x 64 tiles per CU (c3): with more, the halves' extra partial
-// traffic costs what the LayerNorm launches save.  FMLH_PREFILL_FUSED=0 turns it off, =1 on.
+// grid has fewer than two 64 x 64 tiles per CU (c3), and at least half of one: with more, the
+// halves' extra partial traffic costs what the LayerNorm launches save.  FMLH_PREFILL_FUSED=0 turns it off, =1 on.
 bool prefill_fused(const fmlh_nanollm* m, int M) {
     const int C = m->C;
     const char* e = std::getenv("FMLH_PREFILL_FUSED");
     if (e && e[0] == '0') return false;
     if (C > 64 * kRowNE || C % 32 != 0) return false;
     const long tiles = (long)((M + 63) / 64) * ((C + 63) / 64);
-    if (!(e && e[0] == '1') && tiles >= 2L * cu_count()) return false;
+    if (2 * tiles < cu_count() || (!(e && e[0] == '1') && tiles >= 2L * cu_count())) return false;
     GemmArgs g;
     g.A = m->y; g.lda = C; g.B = m->layers[0].wproj; g.ldb = C; g.b_trans = 1; g.M = M; g.N = C; g.K = C;
     if (!gemm_runs_nt(g)) return false;
@@ -824,19 +824,20 @@ int prefill_resid_ln(int C, const float* A, const float* W, int K, int M, float*
 }
 
 // Workspace floats one part of a fused prefill takes for Mp rows: the residual projections'
-// two K halves (2 Mp C) or whatever the QKV and FC products plan at Mp rows (a part can be
-// small enough for them to split K), whichever is larger.
-size_t fused_part_ws(const fmlh_nanollm* m, int Mp) {
+// two K halves (2 Mp C) or the QKV and FC products' K ranges as planned for all M rows,
+// whichever is larger.
+size_t fused_part_ws(const fmlh_nanollm* m, int Mp, int M) {
     const int C = m->C;
-    return std::max({(size_t)2 * Mp * C, plan_gemm(Mp, 3 * C, C, 1).ws_elems, plan_gemm(Mp, 4 * C, C, 1).ws_elems});
+    return (size_t)Mp * C * std::max({2, 3 * plan_gemm(M, 3 * C, C, 1).splits, 4 * plan_gemm(M, 4 * C, C, 1).splits});
 }
 
 // Layer l (l = -1: LN0 of layer 0) of a fused prefill (prefill_fused) for sequences b0 ..
-// b0 + nb - 1 of P rows each, on stream s, with ws (ws_cap >= fused_part_ws(m, nb P) floats)
-// for the partial sums: the rows, cache entries and partials of these sequences only, so
+// b0 + nb - 1 of P rows each, of plan_rows rows in all (what the products are planned for), on
+// stream s, with ws (ws_cap >= fused_part_ws(m, nb P, plan_rows) floats) for the partial sums: the rows, cache entries and partials of these sequences only, so
 // disjoint ranges can run on different streams at once.  x holds the embeddings before layer
 // -1; xn holds ln_f(x) of every row after the last layer.
-int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, hipStream_t s, float* ws, size_t ws_cap) {
+int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, int plan_rows, hipStream_t s, float* ws,
+                       size_t ws_cap) {
     const int C = m->C, M = nb * P;
     const size_t r0 = (size_t)b0 * P;
     float* x = m->x + r0 * C;
@@ -853,7 +854,7 @@ int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, hipStream_
         float* vc = m->vc + lofs + kv0;
         GemmArgs g;
         g.A = xn; g.lda = C; g.B = w.wqkvT; g.ldb = C; g.b_trans = 1;
-        g.C = qkv; g.ldc = 3 * C; g.M = M; g.N = 3 * C; g.K = C; g.s = s;
+        g.C = qkv; g.ldc = 3 * C; g.M = M; g.N = 3 * C; g.K = C; g.plan_rows = plan_rows; g.s = s;
         if (gemm_runs_nt(g)) {  // K / V columns written straight into the caches
             g.epi = kEpiKV;
             g.kv.kc = kc; g.kv.vc = vc; g.kv.C = C; g.kv.H = m->H; g.kv.hd = m->hd; g.kv.T = m->T;
@@ -867,7 +868,8 @@ int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, hipStream_
         FMLH_TRY(prefill_resid_ln(C, y, w.wproj, C, M, x, xn, w.ln1g, w.ln1b, ws, s));
         GemmArgs f;
         f.A = xn; f.lda = C; f.B = w.wfcT; f.ldb = C; f.b_trans = 1;
-        f.C = h; f.ldc = 4 * C; f.M = M; f.N = 4 * C; f.K = C; f.epi = kEpiGelu; f.s = s;
+        f.C = h; f.ldc = 4 * C; f.M = M; f.N = 4 * C; f.K = C; f.epi = kEpiGelu; f.plan_rows = plan_rows;
+        f.s = s;
         FMLH_TRY(gemm(f, ws, ws_cap));
         const bool last = l + 1 == m->L;
         FMLH_TRY(prefill_resid_ln(C, h, w.w2T, 4 * C, M, x, xn, last ? m->lnf_g : m->layers[l + 1].ln0g,
@@ -877,7 +879,7 @@ int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, hipStream_
 }
 
 int prefill_seqs(fmlh_nanollm* m, int b0, int nb, int P, hipStream_t s, float* ws, size_t ws_cap) {
-    for (int l = -1; l < m->L; ++l) FMLH_TRY(prefill_seqs_layer(m, l, b0, nb, P, s, ws, ws_cap));
+    for (int l = -1; l < m->L; ++l) FMLH_TRY(prefill_seqs_layer(m, l, b0, nb, P, nb * P, s, ws, ws_cap));
     return FMLH_OK;
 }
 
@@ -1525,12 +1527,11 @@ int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t
     const int parts = std::min<int>((int)batch, parts_env ? std::max(1, std::min(fmlh_nanollm::kPrefillParts,
                                                                                    std::atoi(parts_env)))
                                                           : 2);
-    // Every part's workspace slice holds what any part plans (a smaller part can plan a split
-    // that a larger one does not: 320 rows of c3's FC product split K, 384 rows do not).
+    // Every part's workspace slice holds what the largest part needs.
     size_t part_ws = 0;
     for (int i = 0; fused && i < parts; ++i) {
         const int nb = (int)batch * (i + 1) / parts - (int)batch * i / parts;
-        part_ws = std::max(part_ws, fused_part_ws(m, nb * (int)P));
+        part_ws = std::max(part_ws, fused_part_ws(m, nb * (int)P, M));
     }
     FMLH_TRY(ensure_ws(m, std::max(gemm_ws_for(m, M), (size_t)parts * part_ws)));
     const size_t n = (size_t)M * m->C;
@@ -1557,7 +1558,7 @@ int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t
         for (int l = -1; l < m->L && rc == FMLH_OK; ++l)  // layer by layer, so every stream has work
             for (int i = 0; i < parts && rc == FMLH_OK; ++i) {
                 const int b0 = (int)batch * i / parts, b1 = (int)batch * (i + 1) / parts;
-                rc = prefill_seqs_layer(m, l, b0, b1 - b0, (int)P, i == 0 ? s : m->s2[i - 1],
+                rc = prefill_seqs_layer(m, l, b0, b1 - b0, (int)P, M, i == 0 ? s : m->s2[i - 1],
                                         m->ws + (size_t)i * part_ws, part_ws);
             }
         // Joined on every path: after a failed launch the library stream still orders the next

@@ -122,6 +122,60 @@ def test_gemm_nt_kernel_tiles(tile, shape, monkeypatch):
     _close(dC.numpy(), acc, 1e-5)
 
 
+# Products on the bf16 matrix cores (operands split into three bf16 parts): one row past a tile,
+# one K block and the remainder of the wide tile's, both tiles and both layouts of B.  Bound:
+# every 8 k of the six part products round once (6 K / 8 roundings of 2^-24 on sums below
+# |A||B|), the parts left out are below 2^-24.
+@pytest.mark.parametrize("tile", ["128x128", "64x64"])
+@pytest.mark.parametrize("bt", [0, 1])
+@pytest.mark.parametrize("shape", [(65, 129, 16), (129, 65, 48), (257, 300, 400), (128, 4096, 16)])
+def test_gemm_split_bf16_edges(shape, bt, tile, monkeypatch):
+    M, N, K = shape
+    print(f"split gemm tile={tile} M={M} N={N} K={K} bt={bt}", flush=True)
+    monkeypatch.setenv("FMLH_GEMM_NT_TILE", tile)
+    r = _rng(M + N + K)
+    A = r.standard_normal((M, K)).astype(np.float32)
+    W = (r.standard_normal((K, N)) * np.exp2(r.integers(-12, 12, (K, N)))).astype(np.float32)
+    dA, dW, dC = D(A), D(np.ascontiguousarray(W.T) if bt else W), fh.DeviceArray((M, N))
+    fh.gemm_ex(dA.ptr, K, dW.ptr, K if bt else N, bt, dC.ptr, N, M, N, K, fh.EPI_NONE, 0, N)
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    err = np.abs(dC.numpy() - A64 @ W64)
+    assert np.all(err <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
+
+
+# Operands the bf16 parts cannot carry take the fp32 path inside the kernel: infinities and NaN
+# give what fp32 arithmetic gives, rows of tiny elements keep their relative accuracy.
+@pytest.mark.parametrize("tile", ["128x128", "64x64"])
+def test_gemm_split_bf16_special_values(tile, monkeypatch):
+    monkeypatch.setenv("FMLH_GEMM_NT_TILE", tile)
+    M, N, K = 300, 200, 96
+    r = _rng(5)
+    A = r.standard_normal((M, K)).astype(np.float32)
+    W = r.standard_normal((K, N)).astype(np.float32)
+    A[3, 7] = np.inf
+    A[150, 0], A[151, 5] = -np.inf, np.nan
+    A[290, 9] = 3.4e38  # rounds to an infinity in bf16
+    W[:, 130] *= np.float32(1e-34)
+    A[70, :] *= np.float32(1e-33)
+    W[7, 11] = 0.0  # infinity times zero
+    dA, dW, dC = D(A), D(W), fh.DeviceArray((M, N))
+    fh.gemm_ex(dA.ptr, K, dW.ptr, N, 0, dC.ptr, N, M, N, K, fh.EPI_NONE, 0, N)
+    got = dC.numpy().astype(np.float64)
+    with np.errstate(all="ignore"):
+        ref = A.astype(np.float64) @ W.astype(np.float64)
+        ref[np.abs(ref) > np.finfo(np.float32).max] = np.inf * np.sign(ref[np.abs(ref) > np.finfo(np.float32).max])
+        prod = np.abs(A.astype(np.float64)) @ np.abs(W.astype(np.float64))
+    # the row whose partial sums lie at the end of fp32's range may overflow either way
+    ok = np.ones((M, N), bool)
+    ok[290] = np.abs(prod[290]) < 1e38
+    fin = np.isfinite(ref) & ok
+    assert np.array_equal(np.isnan(got)[ok], np.isnan(ref)[ok])
+    assert np.array_equal(got[ok & np.isinf(ref)], ref[ok & np.isinf(ref)])
+    # sums below fp32's smallest normal number (1e-34 * 1e-33) are not held to a relative bound
+    err = np.abs(got - ref)[fin]
+    assert np.all(err <= (0.75 * K + 8) * 2.0 ** -24 * prod[fin] + 2.0 ** -126)
+
+
 @pytest.mark.parametrize("epi", [fh.EPI_GELU, fh.EPI_RESID])
 @pytest.mark.parametrize("tile", ["128x128", "64x64"])
 def test_gemm_nt_kernel_epilogues_in_place(epi, tile, monkeypatch):
