@@ -1063,6 +1063,31 @@ int gemm_split_partials(const GemmArgs& g, float* ws, size_t ws_elems, int* spli
     return FMLH_OK;
 }
 
+namespace {
+// Whether a strided product runs on the split bf16 tiles; fills everything but the output.  They
+// take views with a contiguous index on either side from 64 tiles' worth of outputs on: fewer
+// leave CUs idle that the wave-split kernel's 16 x 16 tiles still use (us, that kernel / this one:
+// 24 tiles 256 x 64 x 256 6.1 / 9.1, 16 tiles 256 x 256 x 2048 20 / 48; 64 tiles 512 x 64 x 512 19
+// / 14.8; 192 tiles 1024 x 64 x 1024 41 / 26; 576 tiles 3072 x 768 x 1024 96 / 49).  The small part
+// products are summed apart, which keeps the error below that kernel's four K ranges' (K 1024:
+// 1.9e-7 / 2.9e-7).  128 x 128 tiles from two per CU on (1024 x 1024 x 64, 12 planes: 27.0 / 28.0).
+bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M, uint32_t N, uint32_t K, uint32_t l_rs,
+                   uint32_t l_cs, uint32_t r_rs, uint32_t r_cs, uint32_t o_rs, uint32_t o_cs, uint32_t batch,
+                   size_t l_plane, size_t r_plane, SplitGemm* q) {
+    if (o_cs != 1 || o_rs > INT32_MAX || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || batch > 65535) return false;
+    if ((double)M * N * batch < 64.0 * 64 * 64) return false;
+    // Strides between the k of one row of A (column of B) and between its rows (columns).
+    const uint32_t a_k = tl ? l_rs : l_cs, a_r = tl ? l_cs : l_rs, b_k = tr ? r_cs : r_rs, b_r = tr ? r_rs : r_cs;
+    if ((a_k != 1 && a_r != 1) || (b_k != 1 && b_r != 1)) return false;
+    q->A = L; q->a_kc = a_k == 1; q->lda = (int)std::min<uint32_t>(a_k == 1 ? a_r : a_k, INT32_MAX); q->a_plane = l_plane;
+    q->B = R; q->b_kc = b_k == 1; q->ldb = (int)std::min<uint32_t>(b_k == 1 ? b_r : b_k, INT32_MAX); q->b_plane = r_plane;
+    q->M = (int)M; q->N = (int)N; q->K = (int)K; q->planes = (int)batch;
+    q->low = true;
+    q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * cu_count() ? 128 : 64;
+    return gemm_split_takes(*q);
+}
+}  // namespace
+
 int gemm_strided(int mode, float* out, const float* L, const float* R, uint32_t M, uint32_t N,
                  uint32_t K, uint32_t l_rs, uint32_t l_cs, uint32_t r_rs, uint32_t r_cs,
                  uint32_t o_rs, uint32_t o_cs, uint32_t batch, size_t l_plane, size_t r_plane,
@@ -1070,6 +1095,13 @@ int gemm_strided(int mode, float* out, const float* L, const float* R, uint32_t 
     if (M == 0 || N == 0 || batch == 0) return FMLH_OK;
     const bool tl = mode == FMLH_TRANSPOSE_LEFT || mode == FMLH_TRANSPOSE_BOTH;
     const bool tr = mode == FMLH_TRANSPOSE_RIGHT || mode == FMLH_TRANSPOSE_BOTH;
+    {
+        SplitGemm q;
+        if (strided_split(tl, tr, L, R, M, N, K, l_rs, l_cs, r_rs, r_cs, o_rs, o_cs, batch, l_plane, r_plane, &q)) {
+            q.C = out; q.ldc = (int)o_rs; q.c_plane = o_plane; q.s = s;
+            return gemm_split(q);
+        }
+    }
     // K within one 64-wide chunk: one chunk per 32 x 32 tile.  Longer K: the wave-split
     // kernel, with 16 x 16 tiles unless 32 x 32 tiles already give a work-group per CU.
     const size_t tiles32 = (size_t)((N + 31) / 32) * ((M + 31) / 32) * batch;

@@ -176,6 +176,37 @@ def test_gemm_split_bf16_special_values(tile, monkeypatch):
     assert np.all(err <= (0.75 * K + 8) * 2.0 ** -24 * prod[fin] + 2.0 ** -126)
 
 
+# Strided products of 64 tiles' worth of outputs and more (the split bf16 tiles): every mode, both
+# index orders of each operand (rows or columns contiguous), batched planes, K with a remainder,
+# row strides that keep 16-byte rows and ones that do not (the wave-split kernel), 128-wide tiles.
+@pytest.mark.parametrize("mode", [fh.NONE, fh.RIGHT, fh.LEFT, fh.BOTH])
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("shape", [(190, 333, 37, 5, 3), (190, 333, 37, 5, 2), (129, 65, 100, 33, 0), (300, 260, 20, 86, 4)])
+def test_matmul_strided_split_tiles(shape, swap, mode):
+    M, N, K, planes, pad = shape
+    print(f"strided split mode={mode} swap={swap} {shape}", flush=True)
+    r = _rng(M + K + mode)
+    A = r.standard_normal((planes, M, K)).astype(np.float32)
+    B = r.standard_normal((planes, K, N)).astype(np.float32)
+
+    def stored(X, transposed):  # as (stored array, plane, row stride, column stride) of X's mode view
+        V = np.swapaxes(X, 1, 2) if transposed else X  # the matrix the call names
+        S = np.swapaxes(V, 1, 2) if swap else V         # how it lies in memory
+        ld = S.shape[2] + (-S.shape[2]) % 4 + pad
+        P = np.zeros((planes, S.shape[1], ld), np.float32)
+        P[:, :, :S.shape[2]] = S
+        return P, P.shape[1] * ld, *((1, ld) if swap else (ld, 1))
+
+    L, lp, lrs, lcs = stored(A, mode in (fh.LEFT, fh.BOTH))
+    R, rp, rrs, rcs = stored(B, mode in (fh.RIGHT, fh.BOTH))
+    dL, dR, dO = D(L), D(R), D(np.full((planes, M, N + 3), 7.0, np.float32))
+    fh.matmul_strided(mode, dO.ptr, dL.ptr, dR.ptr, M, N, K, lrs, lcs, rrs, rcs, N + 3, 1, planes, lp, rp, M * (N + 3))
+    got = dO.numpy()
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(got[:, :, :N] - A64 @ B64) <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)))
+    assert np.all(got[:, :, N:] == 7.0)
+
+
 @pytest.mark.parametrize("epi", [fh.EPI_GELU, fh.EPI_RESID])
 @pytest.mark.parametrize("tile", ["128x128", "64x64"])
 def test_gemm_nt_kernel_epilogues_in_place(epi, tile, monkeypatch):
