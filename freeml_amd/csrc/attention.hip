@@ -3,8 +3,8 @@
 // row softmax, Y_h = P V_h).  The reference materialises every T x T score matrix; here no
 // score matrix is stored:
 //   * prefill: one work-group per block of query rows of one (sequence, head) -- 128 rows on
-//     the 32x32x2 matrix cores for head_dim 64, 64 rows on 16x16x4 for head_dim 32, one wave
-//     per lane-row for head_dim 16 -- keys streamed through LDS in 64-key tiles up to the
+//     the bf16 matrix cores (operands split in three) for head_dim 64, 64 rows on 16x16x4 fp32
+//     for head_dim 32, one wave per lane-row for head_dim 16 -- keys streamed through LDS in 64-key tiles up to the
 //     diagonal, online softmax (running max / sum) per query row; work-groups dispatched
 //     longest (latest) query block first;
 //   * decode: one query row per (sequence, head), the cached keys split into 256-position
@@ -14,6 +14,7 @@
 //
 // KV cache layout: [layer][sequence][head][position][head_dim], fp32.
 #include "attention.h"
+#include "bf16_split.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -359,8 +360,6 @@ int kv_scatter(const float* qkv, int qkv_ld, float* kc, float* vc, int rows, int
 namespace {
 
 using f32x4 = __attribute__((ext_vector_type(4))) float;
-using floatx16 = __attribute__((ext_vector_type(16))) float;
-using f32x2 = __attribute__((ext_vector_type(2))) float;
 
 template <int kCtrl>
 __device__ __forceinline__ float row16_move(float v) {
@@ -543,44 +542,43 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(
     }
 }
 
-// ---- prefill, head_dim 64, on v_mfma_f32_32x32x2f32 ----------------------------------------
+// ---- prefill, head_dim 64, on the bf16 matrix cores -----------------------------------------
 //
 // One work-group of 4 waves per 128 query rows of one (sequence, head); wave v owns the 32
 // queries q0 = 128 qb + 32 v .. +31, one per lane column c = lane % 32 (h = lane / 32).  Per
 // 64-key tile up to the diagonal, with the products taken transposed:
-//   S^T (64 keys x 32 queries) = K Q^T       2 blocks of 32 keys x 32 k-steps over the dims
-//   O^T (64 dims x 32 queries) += V^T P^T    2 blocks of 32 dims x 32 k-steps over the keys
-// MFMA 32x32x2 layouts: A (32 x 2) lane supplies A[c][h], B (2 x 32) B[h][c], D (32 x 32)
-// D[8 (r/4) + 4h + r%4][c] in register r.  So lane (h, c) holds, for query c, the scores of
-// keys 32 j + 8 (r/4) + 4h + r%4 (block j, register r) -- half of the tile's keys, the other
-// half in lane c ^ 32.  The row max needs one exchange between the halves; the sum stays a
-// per-lane partial until the end; O^T's registers all belong to query c, so the rescale is
-// lane-local.  Taking the P^T k-step t as key 32 (t/16) + 8 ((t%16)/4) + 4h + t%4 makes
-// register t%16 of score block t/16 exactly lane (h, c)'s B operand: P never leaves registers.
-// The Q k-step t is dim 32h + t (Q row c's half h in 32 registers); row rho of O^T block i
-// is dim 2 rho + i.
-//
-// K and V tiles are copied global -> LDS directly (global_load_lds), two stages: the copy of
-// tile t+1 runs while tile t is multiplied.  Rows are 256 bytes, stored with their 16-byte
-// quads permuted so both read patterns are conflict-free: K (32 lanes read one quad of 32
-// different rows) at quad q ^ (row % 16); V (each half-wave reads a whole key row, 8 bytes
-// per lane, the two halves keys 4 apart) at quad q ^ 8 (key bit 2).  Keys past the work-group's last query copy
-// that query's key row (finite values, masked out).
+//   S^T (64 keys x 32 queries) = K Q^T       2 blocks of 32 keys x 4 k-steps over the dims
+//   O^T (64 dims x 32 queries) += V^T P^T    2 blocks of 32 dims x 4 k-steps over the keys
+// Every operand is split exactly into three bf16 parts (bf16_split.h) and the six part products of
+// weight 2^-16 and more are summed by v_mfma_f32_32x32x16_bf16: ~3100 clocks of a SIMD's matrix
+// core per tile, where the fp32 MFMA needs 8200 (the kernel this one replaced: 540 us per layer
+// at 4 sequences of 3584 rows and 8 heads, now 305; errors against 64 bits level).  The wave's
+// vector work beside them is about as much (softmax, the split of P and of its share of K and V),
+// so two work-groups per CU, out of step, keep both units busy.
+//   * Lane (h, c) of score block j holds, for query c, keys 32 j + 8 (r / 4) + 4 h + r % 4 (register
+//     r) -- half of the tile's keys, the other half in lane c ^ 32.  The row max needs one
+//     exchange between the halves; the sum stays a per-lane partial until the end; O^T's
+//     registers all belong to query c, so the rescale is lane-local.
+//   * Taking keys 16 t + 4 h + {0..3, 8..11} (t = 0, 1) as the 8 k of octet h of P V's k-step t makes
+//     a lane's registers 8 t .. 8 t + 7 its B operand: P is split in registers and never leaves them.
+//   * Q is split once into registers.  K and V tiles go through registers (tile t + 1 is
+//     requested before tile t is multiplied) into one LDS stage of bf16 planes, V transposed:
+//     16-byte units of 8 consecutive dims of a key, and of 8 keys (in the order above) of a dim.
+//     Unit o of row r lies at o ^ (r % 8): any 8 consecutive lanes on one row each, or on one
+//     row's 8 units, touch distinct banks.
+// Infinite keys or values give NaN (their parts are infinity minus infinity), where the products
+// alone would keep some infinities; the LayerNorm behind either makes NaN of both.
 constexpr int kAttnQPerWave = 32;
 constexpr int kAttnQPerWG = 4 * kAttnQPerWave;
-constexpr int kAttnKT = 64;                                        // keys per tile
-constexpr size_t kAttnMfma32Lds = 2 * 2 * kAttnKT * 64 * sizeof(float);  // 2 stages x (K, V)
+constexpr int kAttnKT = 64;  // keys per tile
 
-__device__ __forceinline__ int attn_k_swz(int row) { return row & 15; }
-__device__ __forceinline__ int attn_v_swz(int row) { return ((row >> 2) & 1) << 3; }
-
-__global__ __launch_bounds__(256) void attn_prefill_mfma32_kernel(
+__global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
     const float* __restrict__ qkv, int qkv_ld, const float* __restrict__ kc,
     const float* __restrict__ vc, float* __restrict__ y, int y_ld, int rows_per_seq, int H,
     int T, float scale_log2) {
-    constexpr int HD = 64;
-    constexpr int TILE = kAttnKT * HD;  // floats of one K or V tile
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // [stage][K | V][64][64]
+    constexpr int HD = 64, U = 8;  // 16-byte units per row and plane
+    __shared__ uintx4 kp[3][kAttnKT * U];  // [plane][key][unit]
+    __shared__ uintx4 vp[3][HD * U];       // [plane][dim][unit]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -595,35 +593,59 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma32_kernel(
     const float* kbase = kc + (size_t)bh * T * HD;
     const float* vbase = vc + (size_t)bh * T * HD;
 
-    // Copy assignment: chunk (wave + 4 u) of a tile = rows 4 chunk .. +3; lane -> row
-    // 4 chunk + lane / 16, stored quad lane % 16, which holds global quad (lane % 16) ^ swz(row).
-    const int crow_in = lane >> 4, cpos = lane & 15;
-    auto issue = [&](int tile, int st) {
-        float* kd = lds + st * 2 * TILE;
-        float* vd = kd + TILE;
+    // Staging: K unit u = tid + 256 i is octet u % 8 of key u / 8; V unit u is dim u % 64, keys
+    // 16 (o / 2) + 4 (o % 2) + {0..3, 8..11} of octet o = u / 64.  Keys past the work-group's last
+    // query read that query's row (finite values, masked out).
+    float kv[2][8], vv[2][8];
+    auto load = [&](int tile) {
         const int t0 = tile * kAttnKT;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int chunk = wave + 4 * u;
-            const int row = 4 * chunk + crow_in;
-            const size_t src = (size_t)min(t0 + row, last_q) * HD;
-            copy16_to_lds(kd + chunk * 256, kbase + src + 4 * (cpos ^ attn_k_swz(row)));
-            copy16_to_lds(vd + chunk * 256, vbase + src + 4 * (cpos ^ attn_v_swz(row)));
+        for (int i = 0; i < 2; ++i) {
+            const int u = tid + 256 * i;
+            const float* kr = kbase + (size_t)min(t0 + u / 8, last_q) * HD + 8 * (u % 8);
+            const floatx4 lo = *reinterpret_cast<const floatx4*>(kr);
+            const floatx4 hi = *reinterpret_cast<const floatx4*>(kr + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { kv[i][e] = lo[e]; kv[i][4 + e] = hi[e]; }
+            const int o = u / 64;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = 16 * (o >> 1) + 4 * (o & 1) + (e & 3) + 8 * (e >> 2);
+                vv[i][e] = vbase[(size_t)min(t0 + key, last_q) * HD + u % 64];
+            }
         }
     };
-    issue(0, 0);
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = tid + 256 * i;
+            uintx4 p[3];
+            split8(kv[i], p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) kp[q][(u / 8) * U + ((u % 8) ^ (u / 8 & 7))] = p[q];
+            split8(vv[i], p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) vp[q][(u % 64) * U + ((u / 64) ^ (u & 7))] = p[q];
+        }
+    };
+    load(0);
 
-    // Q^T operand: lane (h, c) holds Q[q0 + c][32h .. 32h + 31] (rows past the sequence read
-    // its last row; their results are not stored).
+    // Q^T operand: lane (h, c) holds dims 16 s + 8 h .. + 7 of query q0 + c (rows past the
+    // sequence read its last row; their results are not stored).
     const bool wave_live = q0 < rows_per_seq;
-    float qv[32];
+    bf16x8 qp[3][4];
     {
         const int qrow = min(q0 + c, rows_per_seq - 1);
-        const float* qp = qkv + ((size_t)b * rows_per_seq + qrow) * qkv_ld + hh * HD + 32 * h;
+        const float* qr = qkv + ((size_t)b * rows_per_seq + qrow) * qkv_ld + hh * HD + 8 * h;
 #pragma unroll
-        for (int t = 0; t < 32; t += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(qp + t);
-            qv[t] = v.x; qv[t + 1] = v.y; qv[t + 2] = v.z; qv[t + 3] = v.w;
+        for (int s = 0; s < 4; ++s) {
+            const floatx4 lo = *reinterpret_cast<const floatx4*>(qr + 16 * s);
+            const floatx4 hi = *reinterpret_cast<const floatx4*>(qr + 16 * s + 4);
+            const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            uintx4 p[3];
+            split8(v, p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) qp[q][s] = __builtin_bit_cast(bf16x8, p[q]);
         }
     }
     floatx16 o[2];
@@ -635,13 +657,13 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma32_kernel(
     const int qpos = q0 + c;
 
     for (int tile = 0; tile < ntiles; ++tile) {
-        // Tile `tile` has landed in every wave's part; all reads of the other stage are done.
-        copies_barrier<0>();
-        if (tile + 1 < ntiles) issue(tile + 1, (tile + 1) & 1);
+        // Every wave has read the tile before; the requested loads stay in flight over a barrier.
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        store();
+        load(min(tile + 1, ntiles - 1));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const int t0 = tile * kAttnKT;
         if (!wave_live || t0 > q0 + kAttnQPerWave - 1) continue;  // no query of the wave sees it
-        const float* ks = lds + (tile & 1) * 2 * TILE;
-        const float* vs = ks + TILE;
 
         // S^T = K Q^T.
         floatx16 s[2];
@@ -651,18 +673,20 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma32_kernel(
             for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {  // quads 8h + u of key rows c and 32 + c
-            f32x4 ka[2];
+        for (int st = 0; st < 4; ++st) {
+            bf16x8 ka[3][2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int row = 32 * j + c;
-                ka[j] = *reinterpret_cast<const f32x4*>(ks + row * HD + 4 * ((8 * h + u) ^ attn_k_swz(row)));
-            }
+            for (int q = 0; q < 3; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+                for (int j = 0; j < 2; ++j) {
+                    const int row = 32 * j + c;
+                    ka[q][j] = __builtin_bit_cast(bf16x8, kp[q][row * U + ((2 * st + h) ^ (row & 7))]);
+                }
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    s[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[j][e], qv[4 * u + e], s[j], 0, 0, 0);
+                    s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[kSplitA[q]][j], qp[kSplitB[q]][st], s[j], 0, 0, 0);
         }
 
         // Online softmax for query c over this lane's 32 keys and the partner half's.
@@ -701,41 +725,43 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma32_kernel(
                 for (int r = 0; r < 16; ++r) o[i][r] *= corr;
         }
 
-        // O^T += V^T P^T: k-step t -> key 32 (t/16) + 8 ((t%16)/4) + 4h + t%4.  Row rho of O^T
-        // block i is dim 2 rho + i, so lane (h, c) takes dims 2c and 2c+1 of a key in one 8-byte
-        // read; a half tile's 16 reads go out before its 32 MFMAs.
+        // O^T += V^T P^T; row rho of O^T block i is dim 32 i + rho.
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            f32x2 va[16];
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int tt = 0; tt < 16; ++tt) {
-                const int key = 32 * j + 8 * (tt >> 2) + 4 * h + (tt & 3);
-                va[tt] = *reinterpret_cast<const f32x2*>(
-                    vs + key * HD + 4 * ((c >> 1) ^ attn_v_swz(key)) + 2 * (c & 1));
+            for (int t = 0; t < 2; ++t) {
+                float pv[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) pv[e] = s[j][8 * t + e];
+                uintx4 pp[3];
+                split8(pv, pp);
+                bf16x8 va[3][2];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int row = 32 * i + c;
+                        va[q][i] = __builtin_bit_cast(bf16x8, vp[q][row * U + ((4 * j + 2 * t + h) ^ (row & 7))]);
+                    }
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            va[kSplitA[q]][i], __builtin_bit_cast(bf16x8, pp[kSplitB[q]]), o[i], 0, 0, 0);
             }
-#pragma unroll
-            for (int tt = 0; tt < 16; ++tt) {
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[tt].x, s[j][tt], o[0], 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[tt].y, s[j][tt], o[1], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);  // LDS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 32, 0);  // MFMA
-        }
     }
     if (!wave_live) return;
     const float inv = 1.0f / (lsum + __shfl_xor(lsum, 32));
     if (qpos < rows_per_seq) {
         float* dst = y + ((size_t)b * rows_per_seq + qpos) * y_ld + hh * HD;
-        // Register r of block i: dim 2 (8 (r/4) + 4h + r%4) + i.
+        // Register r of block i: dim 32 i + 8 (r / 4) + 4 h + r % 4.
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float4 lo = make_float4(o[0][4 * u] * inv, o[1][4 * u] * inv,
-                                          o[0][4 * u + 1] * inv, o[1][4 * u + 1] * inv);
-            const float4 hi = make_float4(o[0][4 * u + 2] * inv, o[1][4 * u + 2] * inv,
-                                          o[0][4 * u + 3] * inv, o[1][4 * u + 3] * inv);
-            *reinterpret_cast<float4*>(dst + 16 * u + 8 * h) = lo;
-            *reinterpret_cast<float4*>(dst + 16 * u + 8 * h + 4) = hi;
-        }
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                *reinterpret_cast<float4*>(dst + 32 * i + 8 * u + 4 * h) =
+                    make_float4(o[i][4 * u] * inv, o[i][4 * u + 1] * inv, o[i][4 * u + 2] * inv, o[i][4 * u + 3] * inv);
     }
 }
 
@@ -747,21 +773,21 @@ int attn_prefill(const float* qkv, int qkv_ld, const float* kc, const float* vc,
                  int y_ld, int batch, int rows_per_seq, int H, int HDv, int T, float scale,
                  hipStream_t s) {
     dim3 grid(batch * H, (rows_per_seq + 63) / 64);
-    // head_dim 64 from 256 rows per sequence on: attn_prefill_mfma32_kernel (interleaved A/B on
-    // MI355X against the 16x16x4 kernel: c5 prefill 5.80 vs 6.16 ms, c4 equal; at 64 rows, half
-    // of its 128-query blocks are empty: 15.1 vs 12.7 us per layer at c3); otherwise the 16x16x4
-    // kernel, which FMLH_ATTN_PREFILL=mfma16 selects for every length and FMLH_ATTN_PREFILL=mfma32
-    // replaces for every head_dim-64 length; FMLH_ATTN_PREFILL=simt: the per-lane kernel (the
-    // one head_dim 16 always uses).  The alternatives serve comparisons.
+    // head_dim 64 from 256 rows per sequence on: attn_prefill_split_kernel (a prefill of 8 x 256
+    // rows, 6 layers of 384: 906 us, 936 with the 16x16x4 kernel; below, its 128-query blocks
+    // leave lanes empty: 64 x 64 rows 1510 against 1430); otherwise the 16x16x4 kernel, which
+    // FMLH_ATTN_PREFILL=mfma16 selects for every length and =mfma32 replaces for every
+    // head_dim-64 length; FMLH_ATTN_PREFILL=simt: the per-lane kernel (the one head_dim 16
+    // always uses).  The alternatives serve comparisons.
     const char* env = std::getenv("FMLH_ATTN_PREFILL");
     const bool simt = env && std::strcmp(env, "simt") == 0;
     const bool mfma16 = env && std::strcmp(env, "mfma16") == 0;
     const bool mfma32 = env && std::strcmp(env, "mfma32") == 0;
     if (HDv == 64 && !simt && !mfma16 && (mfma32 || rows_per_seq >= 256)) {
-        dim3 g32(batch * H, (rows_per_seq + kAttnQPerWG - 1) / kAttnQPerWG);
-        hipLaunchKernelGGL(attn_prefill_mfma32_kernel, g32, dim3(256), kAttnMfma32Lds, s, qkv, qkv_ld,
-                           kc, vc, y, y_ld, rows_per_seq, H, T, scale * 1.4426950408889634f);
-        FMLH_LAUNCHED("attn_prefill_mfma32_kernel");
+        dim3 gs(batch * H, (rows_per_seq + kAttnQPerWG - 1) / kAttnQPerWG);
+        hipLaunchKernelGGL(attn_prefill_split_kernel, gs, dim3(256), 0, s, qkv, qkv_ld, kc, vc, y, y_ld,
+                           rows_per_seq, H, T, scale * 1.4426950408889634f);
+        FMLH_LAUNCHED("attn_prefill_split_kernel");
         return FMLH_OK;
     }
 #define FMLH_PREFILL(HDC)                                                                    \

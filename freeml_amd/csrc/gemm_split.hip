@@ -21,6 +21,7 @@
 // need ~770 clocks, its LDS ~580 (three planes written once, read by two waves) and its
 // vector units ~500 (5.5 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
 // every plane of half as many products) and serve the products with too few large tiles.
+#include "bf16_split.h"
 #include "gemm_split.h"
 
 #include <cstdlib>
@@ -30,33 +31,7 @@ namespace fmlh {
 
 namespace {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ float gelu_ref(float x) { return 0.5f * x * (1.0f + erff(x / 1.41421354f)); }
-
-__device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{x, y}, bf16x2));
-}
-
-// Eight floats -> their three bf16 planes (one 16-byte unit each).
-__device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&p)[3]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float x = v[2 * i], y = v[2 * i + 1];
-        const uint32_t p0 = pack_bf16(x, y);
-        const float rx = x - __uint_as_float(p0 << 16), ry = y - __uint_as_float(p0 & 0xffff0000u);
-        const uint32_t p1 = pack_bf16(rx, ry);
-        const float sx = rx - __uint_as_float(p1 << 16), sy = ry - __uint_as_float(p1 & 0xffff0000u);
-        p[0][i] = p0;
-        p[1][i] = p1;
-        p[2][i] = pack_bf16(sx, sy);
-    }
-}
 
 // Rows whose largest element is below this (and not zero) do not split exactly any more: the
 // third part falls under bf16's smallest normal.
@@ -260,7 +235,6 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
                 }
             }
             if (ks == 0) stage_next();
-            constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
             for (int q = 0; q < 6; ++q)
 #pragma unroll
@@ -268,7 +242,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
 #pragma unroll
                     for (int j = 0; j < NBK; ++j) {
                         Acc& d = LO && q < 5 ? low[LO ? i : 0][LO ? j : 0] : acc[i][j];
-                        d = Mfma<MT>::bf16(a[pa[q]][i], b[pb[q]][j], d);
+                        d = Mfma<MT>::bf16(a[kSplitA[q]][i], b[kSplitB[q]][j], d);
                     }
         }
     };
