@@ -900,19 +900,20 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
     // against 9.1; from 37 tiles or K > 768 on it is behind: 256 x 1152 x 384 11.4 against 10.5).
     if ((M > 64 && !(b_trans && tiles64 <= 36 && K <= 768)) || (b_trans && 2 * tiles64 >= cus)) {
         p.kind = GemmPlan::kSplit;
-        // Tile and K ranges by the time (us) they take on MI355X: a CU multiplies a 128 x 128 x 16
-        // block in 0.64 us whether it holds one work-group or three, a 64 x 64 x 32 one in 0.58
-        // alone and 0.45 among several; K ranges write and read their partials at 4 TB/s, and a
-        // reduction takes 3.5 us and 0.35 per range.
+        // Tile and K ranges by the time (us) they take, fitted on MI355X to 38 shapes x 2 layouts x
+        // 8 choices (2 % behind the best choice on average, 19 % at worst): a CU multiplies a
+        // 128 x 128 x 16 block in 0.62 us whether it holds one work-group or two, a 64 x 64 x 32 one
+        // in 0.56 alone (0.70 with B stored K x N) and 0.40 among several; K ranges write and read
+        // their partials, and the reduction is a launch.
         float best = INFINITY;
         for (int tile : {128, 64})
             for (int sp = 1; sp <= 8; ++sp) {
                 const size_t ws = (size_t)sp * M * N;
                 if (sp > 1 && (one_range || K / sp < 64 || ws > kNoAllocScratchFloats)) break;
                 const float units = (float)(tile == 128 ? tiles128 : tiles64) * sp / cus, kr = (float)K / sp;
-                const float t = (tile == 128 ? std::max(1.0f, units) * kr / 16 * 0.64f
-                                             : std::max(0.58f, 0.45f * units) * kr / 32) +
-                                (sp > 1 ? 3.5f + 0.35f * sp + 2e-6f * ws : 1e-6f * M * N);
+                const float t = (tile == 128 ? std::max(1.0f, units) * kr / 16 * (b_trans ? 0.62f : 0.64f)
+                                             : std::max(b_trans ? 0.56f : 0.70f, 0.40f * units) * kr / 32) +
+                                (sp > 1 ? 3.5f + 0.15f * sp + 1.6e-6f * ws : 1e-6f * M * N);
                 if (t < best) {
                     best = t;
                     p.bm = p.bn = tile;
@@ -1068,9 +1069,8 @@ namespace {
 // take views with a contiguous index on either side from 64 tiles' worth of outputs on: fewer
 // leave CUs idle that the wave-split kernel's 16 x 16 tiles still use (us, that kernel / this one:
 // 24 tiles 256 x 64 x 256 6.1 / 9.1, 16 tiles 256 x 256 x 2048 20 / 48; 64 tiles 512 x 64 x 512 19
-// / 14.8; 192 tiles 1024 x 64 x 1024 41 / 26; 576 tiles 3072 x 768 x 1024 96 / 49).  The small part
-// products are summed apart, which keeps the error below that kernel's four K ranges' (K 1024:
-// 1.9e-7 / 2.9e-7).  128 x 128 tiles from two per CU on (1024 x 1024 x 64, 12 planes: 27.0 / 28.0).
+// / 14.8; 192 tiles 1024 x 64 x 1024 41 / 26; 576 tiles 3072 x 768 x 1024 96 / 49).  The error is below
+// that of that kernel's four K ranges (K 1024: 2.9e-7 / 1.9e-7).  128 x 128 tiles from two per CU on (1024 x 1024 x 64, 12 planes: 27.0 / 28.0).
 bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M, uint32_t N, uint32_t K, uint32_t l_rs,
                    uint32_t l_cs, uint32_t r_rs, uint32_t r_cs, uint32_t o_rs, uint32_t o_cs, uint32_t batch,
                    size_t l_plane, size_t r_plane, SplitGemm* q) {
@@ -1082,7 +1082,6 @@ bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M,
     q->A = L; q->a_kc = a_k == 1; q->lda = (int)std::min<uint32_t>(a_k == 1 ? a_r : a_k, INT32_MAX); q->a_plane = l_plane;
     q->B = R; q->b_kc = b_k == 1; q->ldb = (int)std::min<uint32_t>(b_k == 1 ? b_r : b_k, INT32_MAX); q->b_plane = r_plane;
     q->M = (int)M; q->N = (int)N; q->K = (int)K; q->planes = (int)batch;
-    q->low = true;
     q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * cu_count() ? 128 : 64;
     return gemm_split_takes(*q);
 }

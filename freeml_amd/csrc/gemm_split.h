@@ -28,8 +28,7 @@ struct SplitGemm {
     // go to partial[split][M][N] instead of C, without an epilogue.
     int splits = 1, k_per_split = 0;
     float* partial = nullptr;
-    int tile = 128;    // 128 x 128 or 64 x 64 tiles
-    bool low = false;  // 128: the five small part products summed apart (64 always does)
+    int tile = 128;  // 128 x 128 or 64 x 64 tiles
     hipStream_t s = nullptr;
 };
 

@@ -4,23 +4,28 @@
 // round-to-nearest bf16 of what is left, 3 x 8 significant bits = fp32's 24), and the product
 // takes the six part products whose weight is 2^-16 or more of the whole,
 //   a b ~ a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0),
-// accumulated in fp32 by the bf16 MFMAs, smallest first.  The three left out are below 2^-24 of
-// |a b| together, under the rounding of one fp32 product.
+// accumulated in fp32 by the bf16 MFMAs: a0 b0 in one accumulator, the five small ones, smallest
+// first, in another that is added at the end.  (In one accumulator each of the six MFMAs rounds the
+// whole sum, and those roundings are not quite unbiased: 2-norm error 4.2e-7 instead of 1.6e-7 at K
+// = 768, and a long decode after a prefill came out less exact than on fp32 MFMAs, 4.1e-7 / 2.8e-7.)
+// The three products left out are below 2^-24 of |a b| together, under the rounding of one fp32
+// product.
 //
 // Why: the fp32 MFMA these products ran on reaches 154 TFLOP/s at most on MI355X (100-113 of it
 // in the kernel this one replaced); bf16 runs at 16 times its nominal rate, so six part products
 // are 2.6 times as fast at the nominal peaks.  A large library bf16 product reaches 1218
-// TFLOP/s, a sixth of which is 203: the 128 x 128 tiles reach 200 at 8192^3.  Measured, before ->
-// after (us): 4096 x 3072 x 768 stored N x K 180 -> 105, stored K x N 193 -> 110; 1024 x 50304 x
-// 768 692 -> 442.  Relative error against 64 bits (2-norm, normal operands): K 384 / 768 / 3072
-// 2.9e-7 / 4.2e-7 / 8.7e-7 (fp32 MFMA: 3.5e-7 / 5.0e-7 / 9.9e-7); with the small part products
-// summed apart (LO) 1.1e-7 / 1.6e-7 / 3.4e-7.
+// TFLOP/s, a sixth of which is 203: the 128 x 128 tiles reach 190 at 8192^3.  Measured, before ->
+// after (us): 4096 x 3072 x 768 stored N x K 180 -> 107, 1024 x 50304 x 768 692 -> 452.  Relative
+// error against 64 bits (2-norm, normal operands): K 384 / 768 / 3072 1.1e-7 / 1.6e-7 / 3.4e-7 (fp32
+// MFMA: 3.5e-7 / 5.0e-7 / 9.9e-7).
 //
 // The operands are split while they are staged (registers -> LDS), so fp32 matrices of any
 // layout are read once and nothing is kept.  Per 128 x 128 x 16 block a work-group's matrix cores
 // need ~770 clocks, its LDS ~580 (three planes written once, read by two waves) and its
 // vector units ~500 (5.5 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
-// every plane of half as many products) and serve the products with too few large tiles.
+// every plane of half as many products) and serve the products with too few large tiles.  The
+// launch bounds matter: left alone, the compiler takes 267 registers for the large tile (one wave
+// per SIMD: 4096 x 3072 x 768 125 us instead of 107).
 #include "bf16_split.h"
 #include "gemm_split.h"
 
@@ -65,8 +70,8 @@ struct Mfma<16> {
     }
 };
 
-template <int BM, int BN, int BK, int WVM, int WVN, bool AKC, bool BKC, int EPI, bool SPLIT, bool LO, int MT>
-__global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
+template <int BM, int BN, int BK, int WVM, int WVN, bool AKC, bool BKC, int EPI, bool SPLIT, int MT>
+__global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_kernel(
     const float* __restrict__ A, int lda, size_t a_plane, const float* __restrict__ B, int ldb, size_t b_plane,
     float* C, int ldc, size_t c_plane, int M, int N, int K, const float* R, int ldr, KvDest kv,
     float* __restrict__ partial, int k_per_split, int tiles_m, int tiles_n) {
@@ -189,7 +194,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
         }
     };
 
-    Acc acc[MB][NBK], low[LO ? MB : 1][LO ? NBK : 1];
+    Acc acc[MB][NBK], low[MB][NBK];  // a0 b0; the five small part products
     auto clear = [&]() {
 #pragma unroll
         for (int i = 0; i < MB; ++i)
@@ -199,14 +204,10 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
                 for (int r = 0; r < AR; ++r) acc[i][j][r] = 0.0f;
     };
     clear();
-    if constexpr (LO) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int j = 0; j < NBK; ++j)
-#pragma unroll
-                for (int r = 0; r < AR; ++r) low[i][j][r] = 0.0f;
-    }
+        for (int j = 0; j < NBK; ++j) low[i][j] = acc[i][j];
 
     // Two LDS stages, one barrier per K block: block k + 1 (in registers since the iteration
     // before) is split and written while block k is multiplied, block k + 2 is requested.  The
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
                 for (int i = 0; i < MB; ++i)
 #pragma unroll
                     for (int j = 0; j < NBK; ++j) {
-                        Acc& d = LO && q < 5 ? low[LO ? i : 0][LO ? j : 0] : acc[i][j];
+                        Acc& d = q < 5 ? low[i][j] : acc[i][j];
                         d = Mfma<MT>::bf16(a[kSplitA[q]][i], b[kSplitB[q]][j], d);
                     }
         }
@@ -267,12 +268,10 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
         multiply(0, []() {});
         barrier();
     }
-    if constexpr (LO) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int j = 0; j < NBK; ++j) acc[i][j] += low[i][j];
-    }
+        for (int j = 0; j < NBK; ++j) acc[i][j] += low[i][j];
     // What the split cannot carry -- infinities (and values that round to one in bf16), which
     // leave a NaN in the sums, and rows of tiny elements -- is multiplied again in fp32.
     {
@@ -378,11 +377,11 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_kernel(
     }
 }
 
-template <int BM, int BN, int BK, bool AKC, bool BKC, int EPI, bool SPLIT, bool LO>
+template <int BM, int BN, int BK, bool AKC, bool BKC, int EPI, bool SPLIT>
 int launch(const SplitGemm& g) {
     const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
     constexpr size_t lds = (size_t)2 * 3 * (BM + BN) * BK * sizeof(uint16_t);  // 48 KB
-    hipLaunchKernelGGL((gemm_split_kernel<BM, BN, BK, 2, 2, AKC, BKC, EPI, SPLIT, LO, BM == 128 ? 32 : 16>),
+    hipLaunchKernelGGL((gemm_split_kernel<BM, BN, BK, 2, 2, AKC, BKC, EPI, SPLIT, BM == 128 ? 32 : 16>),
                        dim3((unsigned)tm * tn, 1, SPLIT ? g.splits : g.planes), dim3(256), lds, g.s, g.A, g.lda,
                        g.a_plane, g.B, g.ldb, g.b_plane, g.C, g.ldc, g.c_plane, g.M, g.N, g.K, g.R, g.ldr, g.kv,
                        g.partial, g.k_per_split, tm, tn);
@@ -392,22 +391,19 @@ int launch(const SplitGemm& g) {
 
 template <int BM, int BN, int BK, bool AKC, bool BKC>
 int by_epilogue(const SplitGemm& g) {
-    constexpr bool LO = BM == 64;  // 64 x 64 tiles have the registers for it at no cost
     if constexpr (AKC) {
-        if (LO || !g.low) {
-            if (g.splits > 1) return launch<BM, BN, BK, AKC, BKC, kEpiNone, true, LO>(g);
-            switch (g.epi) {
-                case kEpiGelu: return launch<BM, BN, BK, AKC, BKC, kEpiGelu, false, LO>(g);
-                case kEpiResid: return launch<BM, BN, BK, AKC, BKC, kEpiResid, false, LO>(g);
-                case kEpiKV:
-                    if constexpr (BKC) return launch<BM, BN, BK, AKC, BKC, kEpiKV, false, LO>(g);
-                    break;
-                default: return launch<BM, BN, BK, AKC, BKC, kEpiNone, false, LO>(g);
-            }
+        if (g.splits > 1) return launch<BM, BN, BK, AKC, BKC, kEpiNone, true>(g);
+        switch (g.epi) {
+            case kEpiGelu: return launch<BM, BN, BK, AKC, BKC, kEpiGelu, false>(g);
+            case kEpiResid: return launch<BM, BN, BK, AKC, BKC, kEpiResid, false>(g);
+            case kEpiKV:
+                if constexpr (BKC) return launch<BM, BN, BK, AKC, BKC, kEpiKV, false>(g);
+                break;
+            default: break;
         }
     }
     FMLH_REQUIRE(g.epi == kEpiNone && g.splits == 1, "gemm_split: epilogue %d, %d splits of this layout", g.epi, g.splits);
-    return launch<BM, BN, BK, AKC, BKC, kEpiNone, false, true>(g);
+    return launch<BM, BN, BK, AKC, BKC, kEpiNone, false>(g);
 }
 
 template <int BM, int BN, int BK>
