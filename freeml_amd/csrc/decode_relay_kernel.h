@@ -1052,7 +1052,64 @@ __device__ __forceinline__ void loop_f2h(const RelayArgs& a, const Role& ro, int
     }
 }
 
-// ---- lm: x_L, ln_f, logits, first maximum -> the token, and the next step's x_0 ---------------
+// ---- lm: x_L, ln_f, logits, first maximum or a draw -> the token, and the next step's x_0 ------
+
+// Inclusive prefix sums over a wave's lanes (wave_reduce's DPP steps leave every lane its own).
+__device__ __forceinline__ float wave_scan(float v) {
+    v += dpp_move<0x111, 0xf>(0.0f, v);
+    v += dpp_move<0x112, 0xf>(0.0f, v);
+    v += dpp_move<0x114, 0xf>(0.0f, v);
+    v += dpp_move<0x118, 0xf>(0.0f, v);
+    v += dpp_move<0x142, 0xa>(0.0f, v);
+    return v + dpp_move<0x143, 0xc>(0.0f, v);
+}
+__device__ __forceinline__ float lane63(float v) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Every wave's share of the ranks of the logits lg[0..V): how many of its V / kWaves logits come
+// before logits `lane` and `lane + 64` (larger first, the lower index on ties), to ranks[wave].
+__device__ __forceinline__ void sample_ranks(const float* lg, int V, int (*ranks)[128]) {
+    const int lane = lane_id(), w = wave_id();
+    const uint32_t k0 = float_key(lg[lane < V ? lane : 0]), k1 = float_key(lg[lane + 64 < V ? lane + 64 : 0]);
+    int r0 = 0, r1 = 0;
+    for (int u = V * w / kWaves; u < V * (w + 1) / kWaves; ++u) {
+        const uint32_t ku = float_key(lg[u]);
+        r0 += ku > k0 || (ku == k0 && u < lane) ? 1 : 0;
+        r1 += ku > k1 || (ku == k1 && u < lane + 64) ? 1 : 0;
+    }
+    ranks[w][lane] = r0;
+    ranks[w][lane + 64] = r1;
+}
+
+// The draw of sample_hist_kernel for V <= 128 logits in one wave: weights exp((z - max) /
+// temperature) of the top_k first-ranked logits, the first index whose running sum exceeds
+// u total (the last kept one where rounding leaves none).
+__device__ __forceinline__ int sample_wave(const float* lg, int V, const SampleCfg& cfg, const int (*ranks)[128], float u) {
+    const int lane = lane_id();
+    const bool in0 = lane < V, in1 = lane + 64 < V;
+    const float z0 = in0 ? lg[lane] : -INFINITY, z1 = in1 ? lg[lane + 64] : -INFINITY;
+    const float m = wave_max(fmaxf(z0, z1));
+    bool keep0 = in0, keep1 = in1;
+    if (cfg.top_k > 0 && cfg.top_k < V) {
+        int r0 = 0, r1 = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            r0 += ranks[w][lane];
+            r1 += ranks[w][lane + 64];
+        }
+        keep0 = in0 && r0 < cfg.top_k;
+        keep1 = in1 && r1 < cfg.top_k;
+    }
+    const float w0 = keep0 ? expf((z0 - m) * cfg.inv_temp) : 0.0f, w1 = keep1 ? expf((z1 - m) * cfg.inv_temp) : 0.0f;
+    const float c0 = wave_scan(w0), s0 = lane63(c0);
+    const float c1 = s0 + wave_scan(w1), target = u * lane63(c1);
+    const uint64_t hit0 = __ballot(w0 > 0.0f && c0 > target), hit1 = __ballot(w1 > 0.0f && c1 > target);
+    if (hit0) return __builtin_ctzll(hit0);
+    if (hit1) return 64 + __builtin_ctzll(hit1);
+    const uint64_t any0 = __ballot(w0 > 0.0f), any1 = __ballot(w1 > 0.0f);
+    return any1 ? 127 - __builtin_clzll(any1) : any0 ? 63 - __builtin_clzll(any0) : 0;
+}
 
 // x_0 of sequence b for step `step`: the embedding of `token` plus position row `prow`
 // (Embedding x2 + AddLayer; dropout p = 0), as exchange words.  Threads o < C.
@@ -1063,7 +1120,9 @@ __device__ __forceinline__ void emit_x0(const RelayArgs& a, int b, int step, con
     if (o < C) ll_put(&a.xw[(size_t)b * C + o], tokrow[o] + prow[o], epoch_of(a, step));
 }
 
-template <int NE>
+// SMP: the launch samples (a.sample.on); compiled apart, so that greedy launches keep their code (the
+// branch alone cost 0.7 us of a 48 us step).
+template <int NE, bool SMP>
 __device__ __forceinline__ void loop_lm(const RelayArgs& a, const Role& ro, int r, const floatx4* wr, float* lds,
                                         int s0, int s1, bool prefetch, bool table) {
     constexpr int C = 64 * NE;
@@ -1081,6 +1140,9 @@ __device__ __forceinline__ void loop_lm(const RelayArgs& a, const Role& ro, int 
     if (o < C) poll_issue(px, src(it), 8 * o, epoch_of(a, it.step));
     const LnPost lp = ln_post_setup<NE, kPasses>(wr, s.xn, a.lnf_g, a.lnf_b, a.V);
     float* lg = s.sv;
+    int (*ranks)[128] = reinterpret_cast<int (*)[128]>(s.sv + 128);  // sampling with top_k
+    static_assert(kRelayMaxVocab <= 128 && 128 + kWaves * 128 <= kScratch, "sampling scratch");
+    const bool rank = SMP && a.sample.top_k > 0 && a.sample.top_k < a.V;
     Meter mt;
     while (true) {
         stamp(a, r, it, 0);
@@ -1089,6 +1151,8 @@ __device__ __forceinline__ void loop_lm(const RelayArgs& a, const Role& ro, int 
         const bool more = next_item_of(a, it, s1, first, stride, nx);
         const int pos = a.pos0 + it.step;
         const bool emit = it.step + 1 < a.n_steps;  // the next step's x_0
+        // The draw's uniform, while the row is waited for.
+        const float u = SMP ? sample_uniform(a.sample.seed, it.b, pos + 1) : 0.0f;
         if (it.b == first && emit && o < C) s.posrow[o] = ld1(a.pos_emb + (size_t)(pos + 1) * C + o);
         if (o < C) {
             poll_settle(px, s.flags, a.err);
@@ -1113,18 +1177,27 @@ __device__ __forceinline__ void loop_lm(const RelayArgs& a, const Role& ro, int 
         });
         lds_barrier();
         stamp(a, r, it, 2);
+        if (rank) {
+            sample_ranks(lg, a.V, ranks);
+            lds_barrier();
+        }
         if (wave_id() == 0) {
             const int lane = lane_id();
-            float bv = -INFINITY;
-            int bi = -1;
-            for (int v = lane; v < a.V; v += 64) {
-                if (bi < 0 || lg[v] > bv) {  // strict: the lower index keeps a tie
-                    bv = lg[v];
-                    bi = v;
+            int t;
+            if constexpr (SMP) {
+                t = sample_wave(lg, a.V, a.sample, ranks, u);
+            } else {
+                float bv = -INFINITY;
+                int bi = -1;
+                for (int v = lane; v < a.V; v += 64) {
+                    if (bi < 0 || lg[v] > bv) {  // strict: the lower index keeps a tie
+                        bv = lg[v];
+                        bi = v;
+                    }
                 }
+                float best;
+                t = wave_argmax(bv, bi, best);
             }
-            float best;
-            const int t = wave_argmax(bv, bi, best);
             if (lane == 0) {
                 const int tk = t < 0 ? 0 : t;
                 a.hist[(size_t)it.b * a.HS + pos + 1] = tk;
@@ -1149,7 +1222,7 @@ __device__ __forceinline__ void loop_lm(const RelayArgs& a, const Role& ro, int 
 // ---- role dispatch -----------------------------------------------------------------------------
 
 // Items of steps [s0, s1) of role ro (kind K) with its weights in wr.
-template <int NE, bool QA, bool BIG, int FR, int K>
+template <int NE, bool QA, bool BIG, int FR, bool SMP, int K>
 __device__ __forceinline__ void run_items(const RelayArgs& a, const Role& ro, int r, const floatx4* wr, float* lds,
                                           int s0, int s1, bool single) {
     if constexpr (K == kQ) loop_q<NE, QA, BIG>(a, ro, r, wr, lds, s0, s1, single);
@@ -1157,33 +1230,33 @@ __device__ __forceinline__ void run_items(const RelayArgs& a, const Role& ro, in
     else if constexpr (K == kF) loop_f<NE, BIG, FR>(a, ro, r, wr, lds, s0, s1, single);
     else if constexpr (K == kF2 && FR == kRelayHRows) loop_f2h<NE>(a, ro, r, wr, lds, s0, s1, single);
     else if constexpr (K == kF2) loop_f2<NE, FR>(a, ro, r, lds, s0, s1, single);
-    else loop_lm<NE>(a, ro, r, wr, lds, s0, s1, single, single);
+    else loop_lm<NE, SMP>(a, ro, r, wr, lds, s0, s1, single, single);
 }
 
 // A workgroup with one role: its weights are loaded once, and it runs every item of the launch
 // with the next item's inputs requested early (prefetch).
-template <int NE, bool QA, bool BIG, int FR, int K>
+template <int NE, bool QA, bool BIG, int FR, bool SMP, int K>
 __device__ __forceinline__ void run_single(const RelayArgs& a, const Role& ro, int r, float* lds) {
     floatx4 wr[wr_count<NE, K, QA, BIG, FR>()];
     load_weights<NE, K, QA, BIG, FR>(a, ro, wr);
-    run_items<NE, QA, BIG, FR, K>(a, ro, r, wr, lds, 0, a.n_steps, true);
+    run_items<NE, QA, BIG, FR, SMP, K>(a, ro, r, wr, lds, 0, a.n_steps, true);
 }
 
 // One role of a workgroup with two, for one step: the role's weights are requested when it
 // starts (its inputs come much later: the role before it in the step order is several layers
 // back); its items run without prefetch.
-template <int NE, bool QA, bool BIG, int FR, int K>
+template <int NE, bool QA, bool BIG, int FR, bool SMP, int K>
 __device__ __forceinline__ void run_loaded(const RelayArgs& a, const Role& ro, int r, int step, float* lds) {
     floatx4 wr[wr_count<NE, K, QA, BIG, FR>()];
     load_weights<NE, K, QA, BIG, FR>(a, ro, wr);
-    run_items<NE, QA, BIG, FR, K>(a, ro, r, wr, lds, step, step + 1, false);
+    run_items<NE, QA, BIG, FR, SMP, K>(a, ro, r, wr, lds, step, step + 1, false);
 }
 
 // SPLIT (with BIG): two attention and two lm_head workgroups per head / model, each taking every
 // other sequence, and at n_embed 384 FC slices of kRelaySplitFRows rows (to stay within 256
 // workgroups for six layers); SPLIT 2 (n_embed 384), the h cut: FC slices of kRelayHRows rows
 // that publish h, and the MLP projection's rows in the F2 team.
-template <int NE, bool QA, bool BIG, int SPLIT>
+template <int NE, bool QA, bool BIG, int SPLIT, bool SMP>
 __global__ __launch_bounds__(kThreads) void decode_relay_kernel(RelayArgs a) {
     constexpr int C = 64 * NE, H = C / kHD;
     constexpr int FR = SPLIT == 2 ? kRelayHRows : SPLIT && NE == 6 ? kRelaySplitFRows : kRelayFRows;
@@ -1211,26 +1284,26 @@ __global__ __launch_bounds__(kThreads) void decode_relay_kernel(RelayArgs a) {
     const Role ro = role_of(a, H, w);
     if (w + G >= a.roles) {
         switch (ro.kind) {
-            case kQ: run_single<NE, QA, BIG, FR, kQ>(a, ro, w, lds); break;
-            case kA: run_single<NE, QA, BIG, FR, kA>(a, ro, w, lds); break;
-            case kF: run_single<NE, QA, BIG, FR, kF>(a, ro, w, lds); break;
+            case kQ: run_single<NE, QA, BIG, FR, SMP, kQ>(a, ro, w, lds); break;
+            case kA: run_single<NE, QA, BIG, FR, SMP, kA>(a, ro, w, lds); break;
+            case kF: run_single<NE, QA, BIG, FR, SMP, kF>(a, ro, w, lds); break;
             case kF2:
-                if constexpr (BIG) run_single<NE, QA, BIG, FR, kF2>(a, ro, w, lds);
+                if constexpr (BIG) run_single<NE, QA, BIG, FR, SMP, kF2>(a, ro, w, lds);
                 break;
-            default: run_single<NE, QA, BIG, FR, kLm>(a, ro, w, lds); break;
+            default: run_single<NE, QA, BIG, FR, SMP, kLm>(a, ro, w, lds); break;
         }
     } else {
         for (int step = 0; step < a.n_steps; ++step) {
             for (int r = w; r < a.roles; r += G) {
                 const Role rr = role_of(a, H, r);
                 switch (rr.kind) {
-                    case kQ: run_loaded<NE, QA, BIG, FR, kQ>(a, rr, r, step, lds); break;
-                    case kA: run_loaded<NE, QA, BIG, FR, kA>(a, rr, r, step, lds); break;
-                    case kF: run_loaded<NE, QA, BIG, FR, kF>(a, rr, r, step, lds); break;
+                    case kQ: run_loaded<NE, QA, BIG, FR, SMP, kQ>(a, rr, r, step, lds); break;
+                    case kA: run_loaded<NE, QA, BIG, FR, SMP, kA>(a, rr, r, step, lds); break;
+                    case kF: run_loaded<NE, QA, BIG, FR, SMP, kF>(a, rr, r, step, lds); break;
                     case kF2:
-                        if constexpr (BIG) run_loaded<NE, QA, BIG, FR, kF2>(a, rr, r, step, lds);
+                        if constexpr (BIG) run_loaded<NE, QA, BIG, FR, SMP, kF2>(a, rr, r, step, lds);
                         break;
-                    default: run_loaded<NE, QA, BIG, FR, kLm>(a, rr, r, step, lds); break;
+                    default: run_loaded<NE, QA, BIG, FR, SMP, kLm>(a, rr, r, step, lds); break;
                 }
             }
         }
@@ -1243,7 +1316,7 @@ __global__ __launch_bounds__(kThreads) void decode_relay_kernel(RelayArgs a) {
 
 template <int NE, bool QA, bool BIG, int SPLIT>
 int launch(const RelayArgs& a, const RelayPlan& p, hipStream_t s) {
-    auto kern = decode_relay_kernel<NE, QA, BIG, SPLIT>;
+    auto kern = a.sample.on ? decode_relay_kernel<NE, QA, BIG, SPLIT, true> : decode_relay_kernel<NE, QA, BIG, SPLIT, false>;
     FMLH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(p.smem)));
     if (inject_fault(kFaultLaunch))

@@ -19,6 +19,7 @@
 #include "decode_relay.h"
 #include "decode_wide.h"
 #include "fmlh_internal.h"
+#include "sampling.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -115,30 +116,6 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_hist_kernel(int32_t* __
 // exceeds u * (total), u uniform in [0, 1) from the sequence index, the position being filled
 // and the seed (splitmix64, 24 bits).  Each thread owns a contiguous chunk of the row so the
 // block scans run in index order.
-struct SampleCfg {
-    float inv_temp;
-    int top_k;
-    unsigned long long seed;
-};
-
-__device__ __forceinline__ unsigned long long splitmix64(unsigned long long x) {
-    x += 0x9E3779B97F4A7C15ull;
-    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
-    x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
-    return x ^ (x >> 31);
-}
-
-__device__ __forceinline__ float sample_uniform(unsigned long long seed, int b, int p) {
-    const unsigned long long key = ((unsigned long long)(unsigned)b << 32) | (unsigned)p;
-    return (float)(splitmix64(seed ^ splitmix64(key)) >> 40) * (1.0f / 16777216.0f);
-}
-
-// Order-preserving float -> uint32 (larger float, larger key; -0 and +0 distinct, no NaNs).
-__device__ __forceinline__ uint32_t float_key(float v) {
-    const uint32_t u = __float_as_uint(v);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
 // Exclusive prefix sum over the block's threads in thread order (T = blockDim.x, a multiple of
 // 64); also returns the total.
 template <class V>
@@ -934,6 +911,11 @@ int run_blocks(fmlh_nanollm* m, int batch, int rows, bool decode) {
     return FMLH_OK;
 }
 
+SampleCfg sample_cfg(const fmlh_nanollm* m) {
+    if (!(m->temperature > 0.0f)) return SampleCfg{};
+    return SampleCfg{1.0f / m->temperature, (int)m->top_k, m->seed, true};
+}
+
 // ln_f + lm_head on `batch` rows of `src` (src == nullptr: xn already holds ln_f of them), then
 // the device argmax into the history.
 int head_and_pick(fmlh_nanollm* m, const float* src, int batch, bool decode, int pos_const,
@@ -950,7 +932,7 @@ int head_and_pick(fmlh_nanollm* m, const float* src, int batch, bool decode, int
                       nullptr, 0));
     }
     if (m->temperature > 0.0f) {
-        const SampleCfg cfg{1.0f / m->temperature, (int)m->top_k, m->seed};
+        const SampleCfg cfg = sample_cfg(m);
         hipLaunchKernelGGL(sample_hist_kernel, dim3(batch), dim3(kArgmaxThreads), 0, s, m->hist, m->HS, m->logits,
                            m->V, decode ? m->st : nullptr, pos_const, cfg);
         FMLH_LAUNCHED("sample_hist_kernel");
@@ -1257,12 +1239,12 @@ int wide_steps(fmlh_nanollm* m, uint32_t n_steps, bool capture) {
 
 bool use_grouped(const fmlh_nanollm* m, int batch);
 
-// Whether a batch decodes on the relay kernel: by default wherever it is planned for greedy
-// batches of up to kRelayDefaultMaxBatch sequences of a compiled shape, and above that where
+// Whether a batch decodes on the relay kernel (greedily or sampling): by default wherever it is
+// planned for batches of up to kRelayDefaultMaxBatch sequences of a compiled shape, and above that where
 // the grouped kernel (faster there) does not take the batch; FMLH_RELAY=1 takes it up to
 // kRelayMaxBatch, FMLH_RELAY=0 keeps the persistent and grouped kernels.
 bool use_relay(const fmlh_nanollm* m, int batch) {
-    if (!m->relay || batch < 1 || batch > m->r_bmax || m->temperature != 0.0f) return false;
+    if (!m->relay || batch < 1 || batch > m->r_bmax) return false;
     const char* env = std::getenv("FMLH_RELAY");
     if (env && env[0] == '0') return false;
     if (batch > kRelayDefaultMaxBatch && !(env && env[0] == '1') && use_grouped(m, batch)) return false;
@@ -1304,6 +1286,7 @@ int relay_steps(fmlh_nanollm* m, uint32_t n_steps, bool capture) {
     a.hist_slots = capture ? m->logit_hist_slots : 0;
     a.xw = m->r_x; a.partw = m->r_part; a.qkvw = m->r_qkv; a.dx1w = m->r_dx1; a.xpw = m->r_xp; a.err = m->d_err;
     a.trace = m->r_trace;
+    a.sample = sample_cfg(m);
 
     FMLH_TRY(relay_decode(a, p, m->C, m->hd, stream()));
     m->r_last_roles = p.roles;

@@ -324,8 +324,7 @@ int fmlh_nanollm_read_logits(fmlh_nanollm* m, float* out);
 /* Number of tokens generated so far (per sequence) and current batch. */
 int fmlh_nanollm_status(fmlh_nanollm* m, uint32_t* generated, uint32_t* batch);
 /* Which implementation fmlh_nanollm_decode uses for `batch` sequences: FMLH_DECODE_RELAY
- * (greedy batches of up to 56 sequences of the compiled shapes, 64 with FMLH_RELAY=1,
- * block_size <= 256: one
+ * (batches of up to 64 sequences of the compiled shapes, greedy or sampling, block_size <= 256: one
  * cooperative launch per decode call, each product computed by its own small team of
  * workgroups whose weights stay on the chip, the batch's sequences flowing through the teams
  * as a pipeline; FMLH_RELAY=0 turns it off), FMLH_DECODE_PERSISTENT (one cooperative kernel
@@ -353,7 +352,8 @@ int fmlh_nanollm_decode_path(fmlh_nanollm* m, uint32_t batch, int* path, int* wo
  * exp((z_i - max z) / temperature) over the top_k largest logits (ties at the k-th value go to
  * the lower indices; top_k 0 or >= vocab keeps all), by inverse CDF in index order at u * total,
  * u = (splitmix64(seed ^ splitmix64(sequence << 32 | position)) >> 40) / 2^24 for the position
- * being filled.  Decode then takes the graph path. */
+ * being filled.  Decode then takes the relay kernel where it is planned (its lm_head role draws),
+ * else the graph path. */
 int fmlh_nanollm_set_sampling(fmlh_nanollm* m, float temperature, uint32_t top_k, unsigned long long seed);
 
 /* Convenience: prefill + (n_gen - 1) decode steps; copies tokens (batch x n_gen) and, if

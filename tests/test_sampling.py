@@ -107,6 +107,37 @@ def test_device_draws_follow_the_definition(temperature, top_k, golden):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("vocab,batch,temperature,top_k", [(65, 3, 0.8, 40), (65, 1, 1.1, 0), (33, 2, 0.6, 32), (64, 20, 0.9, 7),
+                                                           (96, 17, 1.5, 95), (96, 4, 0.7, 1), (1, 2, 1.0, 0)])
+def test_relay_draws_follow_the_definition(vocab, batch, temperature, top_k):
+    """Sampling inside the relay kernel (its lm_head role draws): every draw equals the definition
+    applied to that step's logits, for vocabularies within one wave's 64 lanes and beyond, both
+    team cuts, and top_k from 1 to all."""
+    import freeml_amd as fh
+    from freeml_amd import synth
+
+    fh.init(0)
+    w = synth.make_weights(synth.NanoLLMShape(vocab, 64, 256, 4, 2), 5, std=0.1)
+    m = fh.NanoLLM(w, max_batch=batch)
+    prompts = np.stack([synth.prompt_tokens(vocab, 9, 60 + b) for b in range(batch)])
+    try:
+        m.set_sampling(temperature, top_k, seed=99)
+        assert m.decode_path(batch)[0] == "relay"
+        toks, logits = m.generate(prompts, 40, with_logits=True)
+    finally:
+        m.close()
+    checked = 0
+    for b in range(batch):
+        for s in range(40):
+            tok, margin = oracle.sample_token(logits[b, s], temperature, top_k, 99, b, 9 + s)
+            if margin < 1e-5:
+                continue
+            assert toks[b, s] == tok, (b, s)
+            checked += 1
+    assert checked >= 38 * batch
+
+
+@pytest.mark.gpu
 def test_top_k_one_is_greedy_and_zero_temperature_restores_greedy(golden):
     import freeml_amd as fh
     from freeml_amd import synth
