@@ -167,6 +167,7 @@ struct GemmArgs {
 struct GemmPlan {
     enum Kind { kSkinnyNN, kSkinnyNT, kMfma, kSplit } kind = kMfma;
     int bm = 64, bn = 64;
+    int k_groups = 1;  // kSplit, 64 x 64: two groups of waves share the work-group's K range
     int splits = 1, k_per_split = 0;
     size_t ws_elems = 0;
 };

@@ -810,6 +810,7 @@ SplitGemm split_args(const GemmArgs& g, int tile) {
 // A planned split product: one launch, or K ranges and their reduction with the epilogue.
 int run_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
     SplitGemm q = split_args(g, p.bm);
+    q.k_groups = p.k_groups;
     if (p.splits == 1) return gemm_split(q);
     q.epi = kEpiNone; q.splits = p.splits; q.k_per_split = p.k_per_split; q.partial = ws;
     FMLH_TRY(gemm_split(q));
@@ -880,6 +881,10 @@ int launch_nt_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
 
 }  // namespace
 
+// Groups of waves per 64 x 64 tile: two where the launch has at most a work-group per CU and each
+// at least four K blocks.
+static int split_k_groups(float work_groups, int k) { return work_groups <= (float)cu_count() && k >= 128 ? 2 : 1; }
+
 GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
     GemmPlan p;
     if (M <= SK_MAXM) {
@@ -895,40 +900,59 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
     const int cus = cu_count() > 0 ? cu_count() : 256;
     const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    // Split bf16 tiles for everything wider than the batched decode, but for a few N x K products
-    // whose short K ranges gemm_nt_split_kernel holds in LDS at once (256 x 384 x 384: 8.2 us
-    // against 9.1; from 37 tiles or K > 768 on it is behind: 256 x 1152 x 384 11.4 against 10.5).
-    if ((M > 64 && !(b_trans && tiles64 <= 36 && K <= 768)) || (b_trans && 2 * tiles64 >= cus)) {
+    // Split bf16 tiles for everything wider than the batched decode, but for the smallest products,
+    // which the fp32 MFMA kernels' K ranges spread over more CUs or which are over before the
+    // split tiles' longer start is (us, fp32 / split): N x K weights of up to 36 tiles and K 768 on
+    // gemm_nt_split_kernel (256 x 384 x 384 8.2 / 9.1; 256 x 1152 x 384 11.4 / 9.2), K x N ones up
+    // to K 384 (256 x 384 x 384 9.3 / 9.7; 150 x 1024 x 256 8.6 / 8.1), and tiles times K to 4096
+    // (1000 x 256 x 64 4.6 / 5.3).
+    const bool small = (tiles64 <= 36 && K <= (b_trans ? 768 : 384)) || tiles64 * K <= 4096;
+    if ((M > 64 && !small) || (b_trans && 2 * tiles64 >= cus)) {
         p.kind = GemmPlan::kSplit;
         // Tile and K ranges by the time (us) they take, fitted on MI355X to 38 shapes x 2 layouts x
-        // 8 choices (2 % behind the best choice on average, 19 % at worst): a CU multiplies a
+        // 8 choices (3 % behind the best choice on average, 19 % at worst): a CU multiplies a
         // 128 x 128 x 16 block in 0.62 us whether it holds one work-group or two, a 64 x 64 x 32 one
-        // in 0.56 alone (0.70 with B stored K x N) and 0.40 among several; K ranges write and read
-        // their partials, and the reduction is a launch.
+        // in 0.56 alone (0.70 with B stored K x N), 0.40 (0.49) by two groups of waves that share
+        // the K range, and 0.40 among several work-groups; K ranges write and read their partials,
+        // and the reduction is a launch.  Two groups serve products of at most a tile per CU, whose
+        // one wave per SIMD would wait out every latency (256 x 1536 x 384 11.1 -> 9.1, 1024 x 768 x
+        // 768 19.5 -> 14.3).
         float best = INFINITY;
-        for (int tile : {128, 64})
+        const float mn = (float)M * N;
+        for (int tile : {128, 64}) {
+            if (tile == 128 && tiles64 < cus / 2) continue;  // too few large tiles for the device
+            const float tiles = (float)(tile == 128 ? tiles128 : tiles64), cu = (float)cus;
+            const float block = tile == 128 ? (b_trans ? 0.62f / 16 : 0.64f / 16) : (b_trans ? 0.56f / 32 : 0.70f / 32);
             for (int sp = 1; sp <= 8; ++sp) {
-                const size_t ws = (size_t)sp * M * N;
-                if (sp > 1 && (one_range || K / sp < 64 || ws > kNoAllocScratchFloats)) break;
-                const float units = (float)(tile == 128 ? tiles128 : tiles64) * sp / cus, kr = (float)K / sp;
-                const float t = (tile == 128 ? std::max(1.0f, units) * kr / 16 * (b_trans ? 0.62f : 0.64f)
-                                             : std::max(b_trans ? 0.56f : 0.70f, 0.40f * units) * kr / 32) +
-                                (sp > 1 ? 3.5f + 0.15f * sp + 1.6e-6f * ws : 1e-6f * M * N);
+                // K ranges pay while CUs are idle.
+                if (sp > 1 && (one_range || tiles * (sp - 1) >= 2 * cu || K < 64 * sp || sp * mn > kNoAllocScratchFloats)) break;
+                const float wgs = tiles * sp, units = wgs / cu, kr = (float)K / sp;
+                const bool two = tile == 64 && split_k_groups(wgs, (int)kr) == 2;
+                const float t = (tile == 128 ? std::max(1.0f, units) * block
+                                 : two       ? 0.71f * block
+                                             : std::max(block, units * (0.40f / 32))) * kr +
+                                (sp > 1 ? 3.5f + 0.15f * sp + 1.6e-6f * sp * mn : 1e-6f * mn);
                 if (t < best) {
                     best = t;
                     p.bm = p.bn = tile;
                     p.splits = sp;
+                    p.k_groups = two ? 2 : 1;
                 }
             }
+        }
         // FMLH_GEMM_NT_TILE=128x128 | 64x64 forces the tile, FMLH_GEMM_NT_SPLIT_K=n the K ranges
         // (0: one).
         if (const char* e = std::getenv("FMLH_GEMM_NT_TILE")) {
             int bm = 0, bn = 0;
-            if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 && (bm == 128 || bm == 64)) p.bm = p.bn = bm;
+            if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 && (bm == 128 || bm == 64)) {
+                p.bm = p.bn = bm;
+                p.k_groups = bm == 64 ? split_k_groups((float)tiles64 * p.splits, K / p.splits) : 1;
+            }
         }
         if (const char* e = one_range ? nullptr : std::getenv("FMLH_GEMM_NT_SPLIT_K")) p.splits = std::max(1, std::atoi(e));
         if (p.splits > 1) {
-            p.k_per_split = ((K + p.splits - 1) / p.splits + 15) / 16 * 16;
+            const int kb = p.bm == 64 ? 32 : 16;  // whole K blocks of the tile
+            p.k_per_split = ((K + p.splits - 1) / p.splits + kb - 1) / kb * kb;
             p.splits = (K + p.k_per_split - 1) / p.k_per_split;
             p.ws_elems = p.splits > 1 ? (size_t)p.splits * M * N : 0;
         }
@@ -1033,6 +1057,7 @@ int gemm_nt_partials(const GemmArgs& g, int splits, float* ws, size_t ws_elems) 
     if (g.M == 0 || g.N == 0) return FMLH_OK;
     SplitGemm q = split_args(g, 64);
     q.epi = kEpiNone; q.splits = splits; q.k_per_split = g.K / splits; q.partial = ws;
+    q.k_groups = split_k_groups((float)((std::max(g.M, g.plan_rows) + 63) / 64) * ((g.N + 63) / 64) * splits, q.k_per_split);
     if (splits == 1) { q.C = ws; q.ldc = g.N; }
     return gemm_split(q);
 }
@@ -1083,6 +1108,7 @@ bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M,
     q->B = R; q->b_kc = b_k == 1; q->ldb = (int)std::min<uint32_t>(b_k == 1 ? b_r : b_k, INT32_MAX); q->b_plane = r_plane;
     q->M = (int)M; q->N = (int)N; q->K = (int)K; q->planes = (int)batch;
     q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * cu_count() ? 128 : 64;
+    if (q->tile == 64) q->k_groups = split_k_groups((float)((M + 63) / 64) * ((N + 63) / 64) * batch, (int)K);
     return gemm_split_takes(*q);
 }
 }  // namespace

@@ -28,7 +28,8 @@ struct SplitGemm {
     // go to partial[split][M][N] instead of C, without an epilogue.
     int splits = 1, k_per_split = 0;
     float* partial = nullptr;
-    int tile = 128;  // 128 x 128 or 64 x 64 tiles
+    int tile = 128;    // 128 x 128 or 64 x 64 tiles
+    int k_groups = 1;  // 64: waves per work-group twofold, each half on half of K
     hipStream_t s = nullptr;
 };
 

@@ -70,8 +70,8 @@ struct Mfma<16> {
     }
 };
 
-template <int BM, int BN, int BK, int WVM, int WVN, bool AKC, bool BKC, int EPI, bool SPLIT, int MT>
-__global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_kernel(
+template <int BM, int BN, int BK, int WVM, int WVN, int KG, bool AKC, bool BKC, int EPI, bool SPLIT, int MT>
+__global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) void gemm_split_kernel(
     const float* __restrict__ A, int lda, size_t a_plane, const float* __restrict__ B, int ldb, size_t b_plane,
     float* C, int ldc, size_t c_plane, int M, int N, int K, const float* R, int ldr, KvDest kv,
     float* __restrict__ partial, int k_per_split, int tiles_m, int tiles_n) {
@@ -84,9 +84,11 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
     using Acc = typename Mfma<MT>::Acc;
     constexpr int AR = Mfma<MT>::kRegs, KM = Mfma<MT>::kK;
     constexpr int STAGE = 3 * (BM + BN) * U;        // units per LDS stage
-    extern __shared__ __attribute__((aligned(16))) uintx4 lds[];
+    extern __shared__ __attribute__((aligned(16))) uintx4 all_lds[];
 
-    const int tid = threadIdx.x;
+    // KG = 2: two groups of waves, each with half of the K range and its own LDS stages.
+    const int grp_k = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+    const int tid = KG == 1 ? threadIdx.x : threadIdx.x % NT;
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WVN, wn = wave % WVN;
     const int h = lane / MT, c = lane % MT;  // this lane's k octet and row / column of an MFMA
@@ -104,8 +106,12 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
     const int tm = 8 * grp + (t - grp * gsz) % gm, tn = (t - grp * gsz) / gm;
     const int row0 = tm * BM, col0 = tn * BN;
     const int z = blockIdx.z;
-    const int kbeg = SPLIT ? z * k_per_split : 0;
-    const int kend = SPLIT ? min(K, kbeg + k_per_split) : K;
+    const int kbeg_wg = SPLIT ? z * k_per_split : 0;
+    const int kend_wg = SPLIT ? min(K, kbeg_wg + k_per_split) : K;
+    const int k_half = KG == 1 ? 0 : (max(kend_wg - kbeg_wg, 0) + 2 * BK - 1) / (2 * BK) * BK;
+    const int kbeg = kbeg_wg + grp_k * k_half;
+    const int kend = KG == 1 || grp_k ? kend_wg : min(kend_wg, kbeg_wg + k_half);
+    uintx4* lds = all_lds + (size_t)grp_k * 2 * STAGE;
     if constexpr (!SPLIT) {
         A += z * a_plane;
         B += z * b_plane;
@@ -247,36 +253,65 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
                     }
         }
     };
-    const int nk = (kend - kbeg) / BK;
-    if (nk > 0) {
-        load(kbeg, true);
-        store(0);
-        load(kbeg + (nk > 1 ? BK : 0), true);
+    // (KG = 2: the second group's range is never the longer one; every barrier is for both.)
+    const int nk = max(kend - kbeg, 0) / BK;
+    const int nk_all = KG == 1 ? nk : (min(kend_wg, kbeg_wg + k_half) - kbeg_wg) / BK;
+    const bool rest = kbeg + nk * BK < kend;
+    if (nk_all > 0) {
+        if (nk > 0) {
+            load(kbeg, true);
+            store(0);
+            load(kbeg + (nk > 1 ? BK : 0), true);
+        }
         barrier();
-        for (int kb = 0; kb < nk; ++kb) {
-            multiply(kb & 1, [&]() {
-                store((kb + 1) & 1);
-                load(kbeg + min(kb + 2, nk - 1) * BK, true);
-            });
+        for (int kb = 0; kb < nk_all; ++kb) {
+            if (KG == 1 || kb < nk)
+                multiply(kb & 1, [&]() {
+                    store((kb + 1) & 1);
+                    load(kbeg + min(kb + 2, nk - 1) * BK, true);
+                });
             barrier();
         }
     }
-    if (kbeg + nk * BK < kend) {  // the rest of K
-        load(kbeg + nk * BK, false);
-        store(0);
+    if (KG == 2 || rest) {  // the rest of K
+        if (rest) {
+            load(kbeg + nk * BK, false);
+            store(0);
+        }
         barrier();
-        multiply(0, []() {});
+        if (rest) multiply(0, []() {});
         barrier();
     }
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < NBK; ++j) acc[i][j] += low[i][j];
+    if constexpr (KG == 2) {  // the second group's sums to the first
+        float* sums = reinterpret_cast<float*>(all_lds);  // [register][thread]; free since the last barrier
+        if (grp_k == 1) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                    for (int r = 0; r < AR; ++r) sums[((i * NBK + j) * AR + r) * NT + tid] = acc[i][j][r];
+        }
+        __syncthreads();
+        if (grp_k == 0) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                    for (int r = 0; r < AR; ++r) acc[i][j][r] += sums[((i * NBK + j) * AR + r) * NT + tid];
+        }
+        __syncthreads();
+    }
     // What the split cannot carry -- infinities (and values that round to one in bf16), which
     // leave a NaN in the sums, and rows of tiny elements -- is multiplied again in fp32.
     {
-        uint32_t* rmax = reinterpret_cast<uint32_t*>(lds);  // free since the last barrier
-        for (int i = tid; i < BM + BN; i += NT) rmax[i] = 0u;
+        uint32_t* rmax = reinterpret_cast<uint32_t*>(all_lds);  // free since the last barrier
+        for (int i = threadIdx.x; i < BM + BN; i += KG * NT) rmax[i] = 0u;
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NA; ++i) atomicMax(&rmax[a_row[i]], __float_as_uint(amax[i]));
@@ -284,7 +319,7 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
         for (int i = 0; i < NB; ++i) atomicMax(&rmax[BM + b_row[i]], __float_as_uint(bmax[i]));
         __syncthreads();
         bool redo = false;
-        for (int i = tid; i < BM + BN; i += NT) {
+        for (int i = threadIdx.x; i < BM + BN; i += KG * NT) {
             const float v = __uint_as_float(rmax[i]);
             redo |= v > 0.0f && v < kSplitTiny;
         }
@@ -296,9 +331,9 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
                 for (int r = 0; r < AR; ++r) redo |= acc[i][j][r] != acc[i][j][r];
         if (__syncthreads_or(redo)) {
             clear();
-            for (int k = kbeg; k < kend; k += 64 / MT) {
-                const int kk = min(k + h, kend - 1);
-                const bool in = k + h < kend;
+            for (int k = kbeg_wg; k < kend_wg; k += 64 / MT) {
+                const int kk = min(k + h, kend_wg - 1);
+                const bool in = k + h < kend_wg;
                 float av[MB], bv[NBK];
 #pragma unroll
                 for (int i = 0; i < MB; ++i) {
@@ -322,13 +357,14 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
     // kEpiKV: cache offset of each row of the tile, (sequence * H * T + position) * head_dim.
     __shared__ size_t kv_row[EPI == kEpiKV ? BM : 1];
     if constexpr (EPI == kEpiKV) {
-        for (int rr = tid; rr < BM; rr += NT) {
+        for (int rr = threadIdx.x; rr < BM; rr += KG * NT) {
             const int gr = min(row0 + rr, M - 1);
             const int sb = gr / kv.rows_per_seq, p = gr - sb * kv.rows_per_seq;
             kv_row[rr] = ((size_t)sb * kv.H * kv.T + p) * kv.hd;
         }
         __syncthreads();
     }
+    if (KG == 2 && grp_k == 1) return;
 #pragma unroll
     for (int j = 0; j < NBK; ++j) {
         const int gc = col0 + wn * WN + MT * j + c;
@@ -377,39 +413,44 @@ __global__ __launch_bounds__(64 * WVM * WVN, BM == 128 ? 2 : 3) void gemm_split_
     }
 }
 
-template <int BM, int BN, int BK, bool AKC, bool BKC, int EPI, bool SPLIT>
+template <int BM, int BN, int BK, int KG, bool AKC, bool BKC, int EPI, bool SPLIT>
 int launch(const SplitGemm& g) {
     const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
-    constexpr size_t lds = (size_t)2 * 3 * (BM + BN) * BK * sizeof(uint16_t);  // 48 KB
-    hipLaunchKernelGGL((gemm_split_kernel<BM, BN, BK, 2, 2, AKC, BKC, EPI, SPLIT, BM == 128 ? 32 : 16>),
-                       dim3((unsigned)tm * tn, 1, SPLIT ? g.splits : g.planes), dim3(256), lds, g.s, g.A, g.lda,
+    constexpr size_t lds = (size_t)KG * 2 * 3 * (BM + BN) * BK * sizeof(uint16_t);  // 48 KB per group
+    auto kern = gemm_split_kernel<BM, BN, BK, 2, 2, KG, AKC, BKC, EPI, SPLIT, BM == 128 ? 32 : 16>;
+    if constexpr (lds > 64 * 1024) {
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        FMLH_HIP(attr);
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)tm * tn, 1, SPLIT ? g.splits : g.planes), dim3(256 * KG), lds, g.s, g.A, g.lda,
                        g.a_plane, g.B, g.ldb, g.b_plane, g.C, g.ldc, g.c_plane, g.M, g.N, g.K, g.R, g.ldr, g.kv,
                        g.partial, g.k_per_split, tm, tn);
     FMLH_LAUNCHED("gemm_split_kernel");
     return FMLH_OK;
 }
 
-template <int BM, int BN, int BK, bool AKC, bool BKC>
+template <int BM, int BN, int BK, int KG, bool AKC, bool BKC>
 int by_epilogue(const SplitGemm& g) {
     if constexpr (AKC) {
-        if (g.splits > 1) return launch<BM, BN, BK, AKC, BKC, kEpiNone, true>(g);
+        if (g.splits > 1) return launch<BM, BN, BK, KG, AKC, BKC, kEpiNone, true>(g);
         switch (g.epi) {
-            case kEpiGelu: return launch<BM, BN, BK, AKC, BKC, kEpiGelu, false>(g);
-            case kEpiResid: return launch<BM, BN, BK, AKC, BKC, kEpiResid, false>(g);
+            case kEpiGelu: return launch<BM, BN, BK, KG, AKC, BKC, kEpiGelu, false>(g);
+            case kEpiResid: return launch<BM, BN, BK, KG, AKC, BKC, kEpiResid, false>(g);
             case kEpiKV:
-                if constexpr (BKC) return launch<BM, BN, BK, AKC, BKC, kEpiKV, false>(g);
+                if constexpr (BKC) return launch<BM, BN, BK, KG, AKC, BKC, kEpiKV, false>(g);
                 break;
             default: break;
         }
     }
     FMLH_REQUIRE(g.epi == kEpiNone && g.splits == 1, "gemm_split: epilogue %d, %d splits of this layout", g.epi, g.splits);
-    return launch<BM, BN, BK, AKC, BKC, kEpiNone, false>(g);
+    return launch<BM, BN, BK, KG, AKC, BKC, kEpiNone, false>(g);
 }
 
-template <int BM, int BN, int BK>
+template <int BM, int BN, int BK, int KG>
 int by_layout(const SplitGemm& g) {
-    if (g.a_kc) return g.b_kc ? by_epilogue<BM, BN, BK, true, true>(g) : by_epilogue<BM, BN, BK, true, false>(g);
-    return g.b_kc ? by_epilogue<BM, BN, BK, false, true>(g) : by_epilogue<BM, BN, BK, false, false>(g);
+    if (g.a_kc) return g.b_kc ? by_epilogue<BM, BN, BK, KG, true, true>(g) : by_epilogue<BM, BN, BK, KG, true, false>(g);
+    return g.b_kc ? by_epilogue<BM, BN, BK, KG, false, true>(g) : by_epilogue<BM, BN, BK, KG, false, false>(g);
 }
 
 }  // namespace
@@ -426,7 +467,8 @@ bool gemm_split_takes(const SplitGemm& g) {
 int gemm_split(const SplitGemm& g) {
     FMLH_REQUIRE(gemm_split_takes(g), "gemm_split: %dx%dx%d operands not aligned", g.M, g.N, g.K);
     FMLH_REQUIRE(g.splits == 1 || (g.partial && g.k_per_split % 16 == 0), "gemm_split: split K without room");
-    return g.tile == 128 ? by_layout<128, 128, 16>(g) : by_layout<64, 64, 32>(g);
+    if (g.tile == 128) return by_layout<128, 128, 16, 1>(g);
+    return g.k_groups == 2 ? by_layout<64, 64, 32, 2>(g) : by_layout<64, 64, 32, 1>(g);
 }
 
 }  // namespace fmlh

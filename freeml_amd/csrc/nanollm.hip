@@ -789,10 +789,11 @@ bool prefill_fused(const fmlh_nanollm* m, int M) {
 
 // Prefill residual projection in two K halves (partials in ws, 2 M C floats), then
 // x += both halves and xn = LN(x; g, bta), on M rows.
-int prefill_resid_ln(int C, const float* A, const float* W, int K, int M, float* x, float* xn, const float* g,
+int prefill_resid_ln(int C, const float* A, const float* W, int K, int M, int plan_rows, float* x, float* xn, const float* g,
                      const float* bta, float* ws, hipStream_t s) {
     GemmArgs ga;
     ga.A = A; ga.lda = K; ga.B = W; ga.ldb = K; ga.b_trans = 1; ga.M = M; ga.N = C; ga.K = K;
+    ga.plan_rows = plan_rows;
     ga.s = s;
     FMLH_TRY(gemm_nt_partials(ga, 2, ws, (size_t)2 * M * C));
     hipLaunchKernelGGL(resid_ln2_rows_kernel, dim3((M + 3) / 4), dim3(256), 0, s, ws, M, C, x, xn, g, bta);
@@ -842,14 +843,14 @@ int prefill_seqs_layer(fmlh_nanollm* m, int l, int b0, int nb, int P, int plan_r
             FMLH_TRY(kv_scatter(qkv, 3 * C, kc, vc, M, P, C, m->H, m->T, nullptr, 0, s));
         }
         FMLH_TRY(attn_prefill(qkv, 3 * C, kc, vc, y, C, nb, P, m->H, m->hd, m->T, m->scale, s));
-        FMLH_TRY(prefill_resid_ln(C, y, w.wproj, C, M, x, xn, w.ln1g, w.ln1b, ws, s));
+        FMLH_TRY(prefill_resid_ln(C, y, w.wproj, C, M, plan_rows, x, xn, w.ln1g, w.ln1b, ws, s));
         GemmArgs f;
         f.A = xn; f.lda = C; f.B = w.wfcT; f.ldb = C; f.b_trans = 1;
         f.C = h; f.ldc = 4 * C; f.M = M; f.N = 4 * C; f.K = C; f.epi = kEpiGelu; f.plan_rows = plan_rows;
         f.s = s;
         FMLH_TRY(gemm(f, ws, ws_cap));
         const bool last = l + 1 == m->L;
-        FMLH_TRY(prefill_resid_ln(C, h, w.w2T, 4 * C, M, x, xn, last ? m->lnf_g : m->layers[l + 1].ln0g,
+        FMLH_TRY(prefill_resid_ln(C, h, w.w2T, 4 * C, M, plan_rows, x, xn, last ? m->lnf_g : m->layers[l + 1].ln0g,
                                   last ? m->lnf_b : m->layers[l + 1].ln0b, ws, s));
     }
     return FMLH_OK;

@@ -128,7 +128,9 @@ def test_gemm_nt_kernel_tiles(tile, shape, monkeypatch):
 # |A||B|), the parts left out are below 2^-24.
 @pytest.mark.parametrize("tile", ["128x128", "64x64"])
 @pytest.mark.parametrize("bt", [0, 1])
-@pytest.mark.parametrize("shape", [(65, 129, 16), (129, 65, 48), (257, 300, 400), (128, 4096, 16)])
+# (the last four: two groups of waves per tile, with equal, unequal and ragged halves of K)
+@pytest.mark.parametrize("shape", [(65, 129, 16), (129, 65, 48), (257, 300, 400), (128, 4096, 16), (130, 200, 128),
+                                   (70, 150, 160), (200, 96, 1008), (66, 66, 4112)])
 def test_gemm_split_bf16_edges(shape, bt, tile, monkeypatch):
     M, N, K = shape
     print(f"split gemm tile={tile} M={M} N={N} K={K} bt={bt}", flush=True)
@@ -181,7 +183,8 @@ def test_gemm_split_bf16_special_values(tile, monkeypatch):
 # row strides that keep 16-byte rows and ones that do not (the wave-split kernel), 128-wide tiles.
 @pytest.mark.parametrize("mode", [fh.NONE, fh.RIGHT, fh.LEFT, fh.BOTH])
 @pytest.mark.parametrize("swap", [False, True])
-@pytest.mark.parametrize("shape", [(190, 333, 37, 5, 3), (190, 333, 37, 5, 2), (129, 65, 100, 33, 0), (300, 260, 20, 86, 4)])
+@pytest.mark.parametrize("shape", [(190, 333, 37, 5, 3), (190, 333, 37, 5, 2), (129, 65, 100, 33, 0), (300, 260, 20, 86, 4),
+                                   (520, 500, 131, 1, 0), (65, 2100, 205, 2, 1)])
 def test_matmul_strided_split_tiles(shape, swap, mode):
     M, N, K, planes, pad = shape
     print(f"strided split mode={mode} swap={swap} {shape}", flush=True)
