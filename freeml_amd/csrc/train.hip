@@ -49,23 +49,24 @@ __global__ void softmax_backward_kernel(float* out, const float* p, const float*
 
 // LayerNormBackwardsOp, parameter gradients (MatrixBase_Functions.h:595-656): dGamma[c] =
 // sum over rows of dY * xHat (xHat recomputed from `in` when not stored), dBeta[c] = sum dY.
-// One block per 64 columns; each of the block's waves sums a strided subset of the rows in
-// row order and the waves' partial sums are added in wave order.
-constexpr unsigned kLnbWaves = 16;
+// One 1024-thread block per 16 columns: thread (column t % 16, lane row t / 16) sums every 64th row
+// in row order, then the 64 partial sums of a column are added in order through LDS, 16 at a time.
+// Bound by latency: with 64 columns per block (a wave per row) a 384- or 768-wide layer kept 6 or
+// 12 CUs busy, 7.4 us at 256 x 384 and 33 at 1024 x 768; 24 and 48 blocks take 3.2 and 9.0.
+constexpr unsigned kLnbCols = 16, kLnbRows = 64;
 
-__global__ void layernorm_backward_params_kernel(float* __restrict__ dgamma, float* __restrict__ dbeta,
-                                                 const float* __restrict__ dy,
-                                                 const float* __restrict__ xhat,
-                                                 const float* __restrict__ mean_inv,
-                                                 const float* __restrict__ in, uint32_t rows,
-                                                 uint32_t cols) {
-    __shared__ float pg[kLnbWaves][kWave];
-    __shared__ float pb[kLnbWaves][kWave];
-    const uint32_t lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-    const uint32_t c = blockIdx.x * kWave + lane;
+__global__ __launch_bounds__(kLnbCols* kLnbRows) void layernorm_backward_params_kernel(
+    float* __restrict__ dgamma, float* __restrict__ dbeta, const float* __restrict__ dy,
+    const float* __restrict__ xhat, const float* __restrict__ mean_inv, const float* __restrict__ in,
+    uint32_t rows, uint32_t cols) {
+    __shared__ float pg[kLnbRows][kLnbCols + 1];
+    __shared__ float pb[kLnbRows][kLnbCols + 1];
+    const uint32_t cl = threadIdx.x % kLnbCols, rl = threadIdx.x / kLnbCols;
+    const uint32_t c = blockIdx.x * kLnbCols + cl;
     float g = 0.0f, b = 0.0f;
     if (c < cols) {
-        for (uint32_t r = w; r < rows; r += kLnbWaves) {
+#pragma unroll 4
+        for (uint32_t r = rl; r < rows; r += kLnbRows) {
             const size_t i = (size_t)r * cols + c;
             const float d = dy[i];
             const float xh = xhat ? xhat[i] : (in[i] - mean_inv[2 * r]) * mean_inv[2 * r + 1];
@@ -73,14 +74,27 @@ __global__ void layernorm_backward_params_kernel(float* __restrict__ dgamma, flo
             b += d;
         }
     }
-    pg[w][lane] = g;
-    pb[w][lane] = b;
+    pg[rl][cl] = g;
+    pb[rl][cl] = b;
     __syncthreads();
-    if (w == 0 && c < cols) {
+    constexpr uint32_t kStep = 16;  // 64 partials -> 4 -> the sum
+    if (rl < kLnbRows / kStep) {
         float sg = 0.0f, sb = 0.0f;
-        for (uint32_t k = 0; k < kLnbWaves; ++k) {
-            sg += pg[k][lane];
-            sb += pb[k][lane];
+#pragma unroll
+        for (uint32_t k = 0; k < kStep; ++k) {
+            sg += pg[rl * kStep + k][cl];
+            sb += pb[rl * kStep + k][cl];
+        }
+        // a group reads its own 16 rows only, so its first may take the sum
+        pg[rl * kStep][cl] = sg;
+        pb[rl * kStep][cl] = sb;
+    }
+    __syncthreads();
+    if (rl == 0 && c < cols) {
+        float sg = 0.0f, sb = 0.0f;
+        for (uint32_t k = 0; k < kLnbRows; k += kStep) {
+            sg += pg[k][cl];
+            sb += pb[k][cl];
         }
         dgamma[c] = sg;
         if (dbeta) dbeta[c] = sb;
@@ -92,7 +106,10 @@ __global__ void layernorm_backward_params_kernel(float* __restrict__ dgamma, flo
 // dXhat = dY * gamma: dVar = sum(dXhat * diff * -0.5 * invStd3), dMean = sum(dXhat * -invStd)
 // + dVar * -2 * sum(diff) / cols; dX = dXhat * invStd + dVar * 2 * diff / cols + dMean / cols.
 // With mean_inv non-null the row's mean and invStd are also stored there (for the parameter
-// pass when no xHat is kept).
+// pass when no xHat is kept).  NE > 0: rows of up to 64 NE columns are read once into registers, x,
+// dY and gamma together (one memory round trip: 3.0 us at 256 x 384, four in sequence took 7.7);
+// NE = 0: longer rows, a pass over memory per sum.  The sums are the same.
+template <int NE>
 __global__ void layernorm_backward_input_kernel(float* __restrict__ dx, const float* __restrict__ dy,
                                                 const float* __restrict__ in,
                                                 const float* __restrict__ gamma,
@@ -104,35 +121,56 @@ __global__ void layernorm_backward_input_kernel(float* __restrict__ dx, const fl
     const float* x = in + (size_t)row * cols;
     const float* g = dy + (size_t)row * cols;
     const float inv_cols = 1.0f / (float)cols;
+    // Element c = lane + 64 m of the row, in registers or from memory.
+    float vx[NE > 0 ? NE : 1], vg[NE > 0 ? NE : 1];
+    if constexpr (NE > 0) {
+        float gm[NE];
+#pragma unroll
+        for (int m = 0; m < NE; ++m) {
+            const uint32_t c = min(lane + kWave * m, cols - 1);
+            vx[m] = x[c];
+            vg[m] = g[c];
+            gm[m] = gamma[c];
+        }
+#pragma unroll
+        for (int m = 0; m < NE; ++m) vg[m] *= gm[m];
+    }
+    auto each = [&](auto f) {  // f(c, x, dXhat)
+        if constexpr (NE > 0) {
+#pragma unroll
+            for (int m = 0; m < NE; ++m)
+                if (lane + kWave * m < cols) f(lane + kWave * m, vx[m], vg[m]);
+        } else {
+            for (uint32_t c = lane; c < cols; c += kWave) f(c, x[c], g[c] * gamma[c]);
+        }
+    };
     float s = 0.0f;
-    for (uint32_t c = lane; c < cols; c += kWave) s += x[c];
+    each([&](uint32_t, float xv, float) { s += xv; });
     const float mean = wave_sum(s) * inv_cols;
     float q = 0.0f;
-    for (uint32_t c = lane; c < cols; c += kWave) {
-        const float d = x[c] - mean;
+    each([&](uint32_t, float xv, float) {
+        const float d = xv - mean;
         q += d * d;
-    }
+    });
     const float var = wave_sum(q) * inv_cols;
     const float inv_std = 1.0f / sqrtf(var + eps);
     const float inv_std3 = inv_std * inv_std * inv_std;
     float dvar = 0.0f, dmean = 0.0f, sdiff = 0.0f;
-    for (uint32_t c = lane; c < cols; c += kWave) {
-        const float diff = x[c] - mean;
-        const float dxh = g[c] * gamma[c];
+    each([&](uint32_t, float xv, float dxh) {
+        const float diff = xv - mean;
         dvar += dxh * diff * -0.5f * inv_std3;
         dmean += dxh * -inv_std;
         sdiff += diff;
-    }
+    });
     dvar = wave_sum(dvar);
     dmean = wave_sum(dmean);
     sdiff = wave_sum(sdiff);
     dmean += dvar * -2.0f * sdiff * inv_cols;
     float* o = dx + (size_t)row * cols;
-    for (uint32_t c = lane; c < cols; c += kWave) {
-        const float diff = x[c] - mean;
-        const float dxh = g[c] * gamma[c];
+    each([&](uint32_t c, float xv, float dxh) {
+        const float diff = xv - mean;
         o[c] = dxh * inv_std + dvar * 2.0f * diff * inv_cols + dmean * inv_cols;
-    }
+    });
     if (mean_inv && lane == 0) {
         mean_inv[2 * row] = mean;
         mean_inv[2 * row + 1] = inv_std;
@@ -228,11 +266,16 @@ __device__ bool cce_target(const float* target, uint32_t steps, uint32_t target_
     return idx != -1;
 }
 
-__global__ void cce_index_kernel(float* __restrict__ grad, float* __restrict__ row_loss,
+// NE > 0: the row (vocab <= NE blockDim) is read once and stays in registers, each exponential formed
+// once; NE = 0: longer rows, a pass over memory each for the maximum, the sum and the gradient.  At
+// 1024 rows of 50304 the three passes took 303 us, one takes 125 (412 MB at 3.3 TB/s; a large copy
+// reaches 4.9: one block fills a CU, so its load, exponentials and store do not overlap another's).
+template <int NE, int THREADS>
+__global__ __launch_bounds__(THREADS) void cce_index_kernel(float* __restrict__ grad, float* __restrict__ row_loss,
                                  const float* __restrict__ target, const float* __restrict__ logits,
                                  uint32_t vocab, uint32_t steps, uint32_t batch,
                                  uint32_t target_batch) {
-    __shared__ float sh[kThreads / kWave];
+    __shared__ float sh[THREADS / kWave];
     __shared__ uint32_t valid_sh;
     const uint32_t row = blockIdx.x;
     const float* z = logits + (size_t)row * vocab;
@@ -255,19 +298,44 @@ __global__ void cce_index_kernel(float* __restrict__ grad, float* __restrict__ r
         if (row_loss && threadIdx.x == 0) row_loss[row] = 0.0f;
         return;
     }
+    float e[NE > 0 ? NE : 1];
     float m = -INFINITY;
-    for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) m = fmaxf(m, z[c]);
+    if constexpr (NE > 0) {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            // uniform base, the thread's offset: no address register per value
+            e[i] = (int)threadIdx.x < (int)vocab - i * THREADS ? (z + i * THREADS)[threadIdx.x] : -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < NE; ++i) m = fmaxf(m, e[i]);
+    } else {
+        for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) m = fmaxf(m, z[c]);
+    }
     m = block_max(m, sh);
     float s = 0.0f;
-    for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) s += expf(z[c] - m);
+    if constexpr (NE > 0) {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            e[i] = expf(e[i] - m);  // past the row: exp(-inf) = 0
+            s += e[i];
+        }
+    } else {
+        for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) s += expf(z[c] - m);
+    }
     s = block_sum(s, sh);
     if (grad) {
         const uint32_t valid = valid_sh;
         const float inv_valid = valid > 0 ? 1.0f / (float)valid : 0.0f;
-        for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) {
-            const float p = expf(z[c] - m) / s;
-            const float ti = (uint32_t)idx == c ? 1.0f : 0.0f;
-            grad[(size_t)row * vocab + c] = (ti - p) * inv_valid;
+        float* g = grad + (size_t)row * vocab;
+        auto value = [&](bool target, float ex) { return ((target ? 1.0f : 0.0f) - ex / s) * inv_valid; };
+        if constexpr (NE > 0) {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                if ((int)threadIdx.x < (int)vocab - i * THREADS)
+                    (g + i * THREADS)[threadIdx.x] = value((int)threadIdx.x == idx - i * THREADS, e[i]);
+            }
+        } else {
+            for (uint32_t c = threadIdx.x; c < vocab; c += blockDim.x) g[c] = value((uint32_t)idx == c, expf(z[c] - m));
         }
     }
     if (row_loss && threadIdx.x == 0) row_loss[row] = (m + logf(s)) - z[idx];
@@ -512,11 +580,16 @@ int fmlh_layernorm_backward(float* dx, const float* dy, const float* in, const f
     }
     float* mean_inv = xhat ? nullptr : ws;
     const unsigned waves = 4;
-    hipLaunchKernelGGL(layernorm_backward_input_kernel, dim3((rows + waves - 1) / waves),
-                       dim3(waves * kWave), 0, stream(), dx, dy, in, gamma, mean_inv, rows, cols, eps);
+#define FMLH_LNB(NE)                                                                                        \
+    hipLaunchKernelGGL(layernorm_backward_input_kernel<NE>, dim3((rows + waves - 1) / waves), dim3(waves * kWave), \
+                       0, stream(), dx, dy, in, gamma, mean_inv, rows, cols, eps)
+    if (cols <= 8 * kWave) FMLH_LNB(8);
+    else if (cols <= 16 * kWave) FMLH_LNB(16);
+    else FMLH_LNB(0);
+#undef FMLH_LNB
     FMLH_LAUNCHED("layernorm_backward_input_kernel");
-    hipLaunchKernelGGL(layernorm_backward_params_kernel, dim3((cols + kWave - 1) / kWave),
-                       dim3(kLnbWaves * kWave), 0, stream(), dgamma, dbeta, dy, xhat, mean_inv, in,
+    hipLaunchKernelGGL(layernorm_backward_params_kernel, dim3((cols + kLnbCols - 1) / kLnbCols),
+                       dim3(kLnbCols * kLnbRows), 0, stream(), dgamma, dbeta, dy, xhat, mean_inv, in,
                        rows, cols);
     FMLH_LAUNCHED("layernorm_backward_params_kernel");
     return FMLH_OK;
@@ -565,8 +638,16 @@ int fmlh_cce_logits(float* grad, float* loss, float* ws, const float* target, co
     }
     float* row_loss = loss ? ws : nullptr;
     if (target_cols == 1) {
-        hipLaunchKernelGGL(cce_index_kernel, dim3(rows), dim3(kThreads), 0, stream(), grad, row_loss,
-                           target, logits, vocab, steps, batch, target_batch);
+#define FMLH_CCE(NE, THREADS)                                                                              \
+    hipLaunchKernelGGL((cce_index_kernel<NE, THREADS>), dim3(rows), dim3(THREADS), 0, stream(), grad, row_loss, target, logits, \
+                       vocab, steps, batch, target_batch)
+        // Rows in registers: up to 16 values per thread of 256, 32 of 1024 (128 registers), 128 of 512.
+        if (vocab <= 4 * 256) FMLH_CCE(4, 256);
+        else if (vocab <= 16 * 256) FMLH_CCE(16, 256);
+        else if (vocab <= 32 * 1024) FMLH_CCE(32, 1024);
+        else if (vocab <= 128 * 512) FMLH_CCE(128, 512);
+        else FMLH_CCE(0, kThreads);
+#undef FMLH_CCE
         FMLH_LAUNCHED("cce_index_kernel");
     } else {
         hipLaunchKernelGGL(cce_onehot_kernel, dim3(rows), dim3(kThreads), 0, stream(), grad,

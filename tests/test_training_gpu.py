@@ -138,6 +138,19 @@ def test_merge_qkv_bit_exact():
     np.testing.assert_array_equal(dp.numpy(), oracle.merge_qkv(q, k, v))
 
 
+# Rows held in registers: the widest of each register count and one more, LayerNorm rows of 8 and 16
+# values per lane and longer ones, one row, and rows around the 64 a block's lanes take at once.
+@pytest.mark.parametrize("rows,cols", [(63, 512), (65, 513), (64, 1024), (3, 1025), (1, 17)])
+def test_layernorm_backward_register_rows(rows, cols):
+    test_layernorm_backward(rows, cols, True, True)
+    test_layernorm_backward(rows, cols, False, True)
+
+
+@pytest.mark.parametrize("vocab", [1, 1024, 1025, 4096, 4097, 32768, 32769, 65536, 65537])
+def test_cce_logits_register_rows(vocab):
+    test_cce_logits("index_ignore", 1, 5, vocab)
+
+
 @pytest.mark.parametrize("kind,batch,steps,vocab",
                          [("index", 1, 256, 65), ("index_ignore", 1, 64, 65), ("index", 4, 128, 50304),
                           ("onehot", 1, 31, 65), ("index_all_ignored", 1, 8, 65)])
