@@ -1489,7 +1489,9 @@ int decode_steps(fmlh_nanollm* m, uint32_t n_steps, bool capture) {
     return FMLH_OK;
 }
 
-int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t P) {
+// rows_only: the blocks alone (forward_window), xn left holding ln_f of every row; nothing is picked and
+// the caller synchronizes.
+int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t P, bool rows_only = false) {
     hipStream_t s = stream();
     // The pinned staging buffer is free: every call that copies from it ends with a stream
     // synchronization.
@@ -1553,6 +1555,8 @@ int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t
         }
         FMLH_TRY(rc);
     }
+    if (rows_only)
+        return fused ? FMLH_OK : layernorm_rows(m->xn, m->x, m->lnf_g, m->lnf_b, nullptr, M, m->C, 1e-5f, s);
     const size_t nl = (size_t)batch * m->C;
     hipLaunchKernelGGL(last_rows_kernel, dim3(blocks_for(nl, 256, 1024u)), dim3(256), 0, s, m->xlast,
                        fused ? m->xn : m->x, (int)P, m->C, (int)batch);
@@ -1923,13 +1927,16 @@ int fmlh_nanollm_forward_window(fmlh_nanollm* m, const int32_t* ids, uint32_t ba
     FMLH_REQUIRE(batch >= 1 && batch <= (uint32_t)m->Bmax, "batch %u outside [1, %d]", batch, m->Bmax);
     m->prefilled = false;
     const uint32_t T = (uint32_t)m->T;
-    FMLH_TRY(do_prefill(m, ids, batch, T));
-    // Logits for every row: ln_f over all rows, then lm_head on all of them.
-    const int M = (int)(batch * T);
     hipStream_t s = stream();
-    float* all = nullptr;
-    FMLH_TRY(device_malloc(reinterpret_cast<void**>(&all), (size_t)M * m->V * sizeof(float)));
-    int rc = layernorm_rows(m->xn, m->x, m->lnf_g, m->lnf_b, nullptr, M, m->C, 1e-5f, s);
+    int rc = do_prefill(m, ids, batch, T, true);
+    // Logits for every row: lm_head on ln_f of all of them, into the MLP's hidden rows where they
+    // fit (V <= 4 C; beyond it the logits take memory of their own).  C = 384, 6 layers, 8 windows:
+    // 868 -> 799 us, with an allocation and a free per call, the last rows' head and pick, a
+    // second ln_f and the wait between the two halves gone.
+    const int M = (int)(batch * T);
+    const bool fits = m->V <= 4 * m->C;
+    float* all = fits ? m->h : nullptr;
+    if (rc == FMLH_OK && !fits) rc = device_malloc(reinterpret_cast<void**>(&all), (size_t)M * m->V * sizeof(float));
     if (rc == FMLH_OK) {
         GemmArgs g;
         g.A = m->xn; g.lda = m->C; g.B = m->lm; g.ldb = m->C; g.b_trans = 1;
@@ -1942,8 +1949,8 @@ int fmlh_nanollm_forward_window(fmlh_nanollm* m, const int32_t* ids, uint32_t ba
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) rc = hip_fail(e, "forward_window copy", __FILE__, __LINE__);
     }
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(all);
+    (void)hipStreamSynchronize(s);  // on every path: the prompt staging buffer is free again
+    if (!fits) (void)hipFree(all);
     m->prefilled = false;  // the window run is not a loop start
     return rc;
 }
