@@ -33,6 +33,10 @@ int device_malloc(void** p, size_t bytes);
 // device (gemm.hip).  setup_noalloc_scratch resolves its address on `device` (current) at
 // fmlh_init; noalloc_scratch returns it, nullptr before initialisation.
 constexpr size_t kNoAllocScratchFloats = size_t(4) << 20;  // 16 MiB
+// Split-K partials of the engine's products and of fmlh_mul (fmlh_gemm_ex plans as its no-alloc
+// variant does): what the 10 K ranges of a 50304-token lm_head's input gradient (1024 x 768) take,
+// 471 us, and the four of 3885 x 768 x 3072, 118; within 16 MiB 537 and 127.
+constexpr size_t kSplitWsFloats = size_t(16) << 20;  // 64 MiB
 int setup_noalloc_scratch(int device);
 float* noalloc_scratch();
 // Floats of split-K partials gemm() needs for this product (0 when it splits nothing).
@@ -152,6 +156,7 @@ struct GemmArgs {
     // Rows to plan the product for instead of M (0: M): parts of one product then take the same
     // tiles and K ranges, so that a row's result does not depend on how many parts there are.
     int plan_rows = 0;
+    size_t ws_max = kSplitWsFloats;  // most split-K partials to plan for
     // ln_g != nullptr: A holds rows before a LayerNorm (LayerNormOp, eps ln_eps, gamma ln_g,
     // optional beta ln_b) and the product takes the normalised rows.  Skinny NT products only
     // (gemm_takes_ln); no normalised copy is written.
@@ -172,7 +177,7 @@ struct GemmPlan {
     size_t ws_elems = 0;
 };
 // one_range: without splitting K (kEpiKV writes its results as they are).
-GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false);
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false, size_t ws_max = kSplitWsFloats);
 
 // Runs the product.  ws/ws_elems: caller workspace for split partials (must hold
 // plan_gemm(...).ws_elems floats); nullptr uses a process-wide buffer grown on demand, which

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -885,7 +886,7 @@ int launch_nt_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
 // at least four K blocks.
 static int split_k_groups(float work_groups, int k) { return work_groups <= (float)cu_count() && k >= 128 ? 2 : 1; }
 
-GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_max) {
     GemmPlan p;
     if (M <= SK_MAXM) {
         if (b_trans) {
@@ -909,29 +910,34 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
     const bool small = (tiles64 <= 36 && K <= (b_trans ? 768 : 384)) || tiles64 * K <= 4096;
     if ((M > 64 && !small) || (b_trans && 2 * tiles64 >= cus)) {
         p.kind = GemmPlan::kSplit;
-        // Tile and K ranges by the time (us) they take, fitted on MI355X to 38 shapes x 2 layouts x
-        // 8 choices (3 % behind the best choice on average, 19 % at worst): a CU multiplies a
-        // 128 x 128 x 16 block in 0.62 us whether it holds one work-group or two, a 64 x 64 x 32 one
-        // in 0.56 alone (0.70 with B stored K x N), 0.40 (0.49) by two groups of waves that share
-        // the K range, and 0.40 among several work-groups; K ranges write and read their partials,
-        // and the reduction is a launch.  Two groups serve products of at most a tile per CU, whose
-        // one wave per SIMD would wait out every latency (256 x 1536 x 384 11.1 -> 9.1, 1024 x 768 x
-        // 768 19.5 -> 14.3).
+        // Tile and K ranges by the time (us) they take, fitted on MI355X to 266 shapes (256 .. 14336
+        // rows of 384 .. 1024-wide blocks, K to 50304) x 2 layouts x up to 15 choices: 0.5 % behind the
+        // best choice on average, 11 % at worst.  A CU multiplies a 128 x 128 x 16 block in 0.62 us
+        // whether it holds one work-group or two, a 64 x 64 x 32 one in 0.64 alone (0.70 with B stored
+        // K x N), 0.45 (0.50) by two groups of waves that share the K range, and 0.41 among several
+        // work-groups; K ranges write and read their partials, and the reduction is a launch.  What
+        // is left of the last work-group per CU counts half (large tiles: the CUs that have none
+        // leave the others clock and bandwidth) or nearly whole (small ones); without that, 2048 x
+        // 768 x 3072 took 92 us instead of 68, 2500 x 1024 x 4096 163 instead of 126.  Two groups
+        // serve products of at most a tile per CU, whose one wave per SIMD would wait out every
+        // latency (256 x 1536 x 384 11.1 -> 9.1, 1024 x 768 x 768 19.5 -> 14.3).
         float best = INFINITY;
         const float mn = (float)M * N;
         for (int tile : {128, 64}) {
             if (tile == 128 && tiles64 < cus / 2) continue;  // too few large tiles for the device
             const float tiles = (float)(tile == 128 ? tiles128 : tiles64), cu = (float)cus;
-            const float block = tile == 128 ? (b_trans ? 0.62f / 16 : 0.64f / 16) : (b_trans ? 0.56f / 32 : 0.70f / 32);
-            for (int sp = 1; sp <= 8; ++sp) {
+            const float block = tile == 128 ? (b_trans ? 0.62f / 16 : 0.665f / 16) : (b_trans ? 0.64f / 32 : 0.70f / 32);
+            const float last = tile == 128 ? 0.5f : 0.85f;
+            for (int sp : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
                 // K ranges pay while CUs are idle.
-                if (sp > 1 && (one_range || tiles * (sp - 1) >= 2 * cu || K < 64 * sp || sp * mn > kNoAllocScratchFloats)) break;
-                const float wgs = tiles * sp, units = wgs / cu, kr = (float)K / sp;
+                if (sp > 1 && (one_range || tiles * (sp - 1) >= 3 * cu || K < 64 * sp || sp * mn > ws_max)) break;
+                const float wgs = tiles * sp, kr = (float)K / sp;
+                const float units = (1.0f - last) * wgs / cu + last * std::ceil(wgs / cu);
                 const bool two = tile == 64 && split_k_groups(wgs, (int)kr) == 2;
                 const float t = (tile == 128 ? std::max(1.0f, units) * block
                                  : two       ? 0.71f * block
-                                             : std::max(block, units * (0.40f / 32))) * kr +
-                                (sp > 1 ? 3.5f + 0.15f * sp + 1.6e-6f * sp * mn : 1e-6f * mn);
+                                             : std::max(block, units * (0.407f / 32))) * kr +
+                                (sp > 1 ? 4.3f + 0.11f * sp + 1.53e-6f * sp * mn : 1.08e-6f * mn);
                 if (t < best) {
                     best = t;
                     p.bm = p.bn = tile;
@@ -977,7 +983,7 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range) {
 namespace {
 // The plan of a call: that of plan_rows rows where given, with room for the call's own.
 GemmPlan plan_for(const GemmArgs& g) {
-    GemmPlan p = plan_gemm(std::max(g.M, g.plan_rows), g.N, g.K, g.b_trans, g.epi == kEpiKV);
+    GemmPlan p = plan_gemm(std::max(g.M, g.plan_rows), g.N, g.K, g.b_trans, g.epi == kEpiKV, g.ws_max);
     if (g.plan_rows > g.M && p.splits > 1) p.ws_elems = (size_t)p.splits * g.M * g.N;
     return p;
 }
@@ -1193,6 +1199,7 @@ int fmlh_gemm_ex(const float* A, int lda, const float* B, int ldb, int b_trans, 
     GemmArgs g;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.b_trans = b_trans ? 1 : 0;
     g.C = C; g.ldc = ldc; g.M = M; g.N = N; g.K = K; g.epi = epilogue; g.R = R; g.ldr = ldr;
+    g.ws_max = kNoAllocScratchFloats;  // the plan of fmlh_gemm_ex_noalloc, whose results are the same
     g.s = stream();
     return gemm(g, nullptr, 0);
 }
@@ -1213,6 +1220,7 @@ int fmlh_gemm_ex_noalloc(const float* A, int lda, const float* B, int ldb, int b
     GemmArgs g;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.b_trans = b_trans ? 1 : 0;
     g.C = C; g.ldc = ldc; g.M = M; g.N = N; g.K = K; g.epi = epilogue; g.R = R; g.ldr = ldr;
+    g.ws_max = kNoAllocScratchFloats;
     g.s = stream();
     const size_t need = gemm_workspace_elems(g);
     if (need > kNoAllocScratchFloats)

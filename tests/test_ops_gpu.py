@@ -178,6 +178,21 @@ def test_gemm_split_bf16_special_values(tile, monkeypatch):
     assert np.all(err <= (0.75 * K + 8) * 2.0 ** -24 * prod[fin] + 2.0 ** -126)
 
 
+# Many K ranges (up to 16, the last one short or ragged) and partials beyond the no-alloc array
+# (1000 x 770 in 6 or more ranges).  Bound: as above, and one rounding per range.
+@pytest.mark.parametrize("mode", [fh.NONE, fh.RIGHT])
+@pytest.mark.parametrize("shape", [(65, 129, 8208), (130, 96, 5008), (1000, 770, 5008), (257, 770, 20016)])
+def test_mul_many_k_ranges(shape, mode):
+    M, N, K = shape
+    print(f"mul mode={mode} {shape}", flush=True)
+    r = _rng(M + N)
+    A, W = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    dA, dW, dC = D(A), D(np.ascontiguousarray(W.T) if mode == fh.RIGHT else W), fh.DeviceArray((M, N))
+    fh.mul(mode, dC.ptr, dA.ptr, dW.ptr, M, N, K)
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    assert np.all(np.abs(dC.numpy() - A64 @ W64) <= (0.75 * K + 24) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
+
+
 # Strided products of 64 tiles' worth of outputs and more (the split bf16 tiles): every mode, both
 # index orders of each operand (rows or columns contiguous), batched planes, K with a remainder,
 # row strides that keep 16-byte rows and ones that do not (the wave-split kernel), 128-wide tiles.
