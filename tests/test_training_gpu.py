@@ -25,6 +25,8 @@ from freeml_amd import checkpoint, synth
 from freeml_amd.dropin import DROPIN, read_train, write_params
 
 pytestmark = pytest.mark.gpu
+# The comparisons with the reference's own training step run its code (test_dropin.py skips likewise).
+needs_dropin = pytest.mark.skipif(not os.path.exists(DROPIN), reason="drop-in driver not built")
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -284,6 +286,7 @@ def train(backend, name, iters, tmp, *extra, env=None):
     return losses, copies
 
 
+@needs_dropin
 @pytest.mark.parametrize("name,iters,per_head", [("c1", 12, False), ("c2", 4, False), ("c2", 4, True)])
 def test_training_iterations_match_reference(name, iters, per_head, tmp_path):
     """K iterations of TrainLoop's step (window + shifted target, forward, CCE gradient,
@@ -308,6 +311,7 @@ def _walk(rec, prefix=""):
         yield from _walk(sub, f"{prefix}{rec.name}/{k}:")
 
 
+@needs_dropin
 @pytest.mark.parametrize("name", ["c1", "c2"])
 def test_backward_gradients_match_reference(name, tmp_path):
     """One backward without optimiser on each backend, saved with Model::Save: every weight
@@ -349,6 +353,7 @@ def test_dropout_mask_bit_exact(n, start, prob):
     np.testing.assert_array_equal(dM.numpy(), oracle.dropout_mask(n, u, start, prob)[0])
 
 
+@needs_dropin
 def test_training_with_biases_and_dropout_matches_reference(tmp_path):
     """The reference's training step with use_bias = true (Dense biases, their SumColumns
     gradient) and dropout 0.1 (embedding, attention-residual and MLP dropout; masks drawn on the
