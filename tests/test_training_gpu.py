@@ -140,6 +140,28 @@ def test_merge_qkv_bit_exact():
     np.testing.assert_array_equal(dp.numpy(), oracle.merge_qkv(q, k, v))
 
 
+# merge_qkv: four columns of a head per thread where head_dim and every pointer allow it: one and several
+# passes of the block over a row, head_dims of 4 and not, and a pointer off by one float.
+@pytest.mark.parametrize("heads,tokens,hd", [(1, 1, 4), (3, 33, 64), (12, 5, 64), (5, 7, 3), (2, 9, 600)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_split_and_merge_qkv_bit_exact(heads, tokens, hd, off):
+    r, C = rng(heads + tokens), heads * hd
+    print(f"split / merge qkv heads={heads} tokens={tokens} hd={hd} offset={off}", flush=True)
+    q, k, v = (r.standard_normal((heads, tokens, hd)).astype(np.float32) for _ in range(3))
+    dq, dk, dv = dev(np.concatenate([np.zeros(off, np.float32), q.ravel()])), dev(k), dev(v)
+    dp = fh.DeviceArray((tokens, 3 * C))
+    fh.merge_qkv(dp.ptr, dq.ptr + 4 * off, dk.ptr, dv.ptr, hd, tokens, heads)
+    rows = [np.ascontiguousarray(t.transpose(1, 0, 2).reshape(tokens, C)) for t in (q, k, v)]
+    np.testing.assert_array_equal(dp.numpy(), np.concatenate(rows, 1))
+    sq, sk, sv = dev(np.full(tokens * C + off, 7.0, np.float32)), fh.DeviceArray((tokens, C)), fh.DeviceArray((tokens, C))
+    fh.split_qkv(sq.ptr + 4 * off, sk.ptr, sv.ptr, dp.ptr, tokens, C)
+    got = sq.numpy()
+    np.testing.assert_array_equal(got[off:].reshape(tokens, C), rows[0])
+    assert np.all(got[:off] == 7.0)
+    np.testing.assert_array_equal(sk.numpy(), rows[1])
+    np.testing.assert_array_equal(sv.numpy(), rows[2])
+
+
 # Rows held in registers: the widest of each register count and one more, LayerNorm rows of 8 and 16
 # values per lane and longer ones, one row, and rows around the 64 a block's lanes take at once.
 @pytest.mark.parametrize("rows,cols", [(63, 512), (65, 513), (64, 1024), (3, 1025), (1, 17)])
