@@ -179,6 +179,11 @@ struct GemmPlan {
 // one_range: without splitting K (kEpiKV writes its results as they are).
 GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false, size_t ws_max = kSplitWsFloats);
 
+// Split-K workspace of an engine step on `rows` rows of each of `batch` sequences: the blocks'
+// products on all of them, the lm_head's on the sequences' last rows.  (Fewer rows can plan more K
+// ranges, so neither number of rows stands in for the other.)
+size_t engine_workspace_elems(int C, int V, int batch, int rows);
+
 // Runs the product.  ws/ws_elems: caller workspace for split partials (must hold
 // plan_gemm(...).ws_elems floats); nullptr uses a process-wide buffer grown on demand, which
 // callers that capture HIP graphs must avoid.

@@ -882,9 +882,12 @@ int launch_nt_split(const GemmArgs& g, const GemmPlan& p, float* ws) {
 
 }  // namespace
 
+// CUs to plan for (no device, as in the host-only tests of the plans: an MI355X's).
+static int plan_cus() { return cu_count() > 0 ? cu_count() : 256; }
+
 // Groups of waves per 64 x 64 tile: two where the launch has at most a work-group per CU and each
 // at least four K blocks.
-static int split_k_groups(float work_groups, int k) { return work_groups <= (float)cu_count() && k >= 128 ? 2 : 1; }
+static int split_k_groups(float work_groups, int k) { return work_groups <= (float)plan_cus() && k >= 128 ? 2 : 1; }
 
 GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_max) {
     GemmPlan p;
@@ -898,7 +901,7 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_m
         }
         return p;
     }
-    const int cus = cu_count() > 0 ? cu_count() : 256;
+    const int cus = plan_cus();
     const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
     // Split bf16 tiles for everything wider than the batched decode, but for the smallest products,
@@ -997,6 +1000,12 @@ bool gemm_runs_nt(const GemmArgs& g) {
     const bool vec_ok = aligned16(g.A) && aligned16(g.B) && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
                         g.K % KB == 0;
     return vec_ok && g.M > 0 && g.N > 0 && g.b_trans && plan_for(g).kind == GemmPlan::kSplit;
+}
+
+size_t engine_workspace_elems(int C, int V, int batch, int rows) {
+    const int M = batch * rows;
+    return std::max({plan_gemm(M, 3 * C, C, 1).ws_elems, plan_gemm(M, C, C, 1).ws_elems, plan_gemm(M, 4 * C, C, 1).ws_elems,
+                     plan_gemm(M, C, 4 * C, 1).ws_elems, plan_gemm(batch, V, C, 1).ws_elems});
 }
 
 size_t gemm_workspace_elems(const GemmArgs& g) {
@@ -1276,6 +1285,19 @@ float* noalloc_scratch() {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     if (stream() == nullptr || g_scratch_device < 0) return nullptr;  // not initialised
     return g_scratch_ptr[g_scratch_device];
+}
+
+// ---- plans, for tests (no device needed) ----------------------------------------------------
+
+extern "C" int fmlh_internal_plan(int M, int N, int K, int b_trans, int* kind, int* tile, int* k_groups, int* splits,
+                                  size_t* ws_elems) {
+    const GemmPlan p = plan_gemm(M, N, K, b_trans);
+    *kind = p.kind; *tile = p.bm; *k_groups = p.k_groups; *splits = p.splits; *ws_elems = p.ws_elems;
+    return FMLH_OK;
+}
+
+extern "C" size_t fmlh_internal_engine_workspace(int C, int V, int batch, int rows) {
+    return engine_workspace_elems(C, V, batch, rows);
 }
 
 void release_global_workspace() {

@@ -646,17 +646,8 @@ void release(fmlh_nanollm* m) {
     }
 }
 
-// Split-K workspace for the five projections at M rows.
-size_t gemm_ws_for(const fmlh_nanollm* m, int M) {
-    const int C = m->C;
-    size_t w = 0;
-    w = std::max(w, plan_gemm(M, 3 * C, C, 1).ws_elems);
-    w = std::max(w, plan_gemm(M, C, C, 1).ws_elems);
-    w = std::max(w, plan_gemm(M, 4 * C, C, 1).ws_elems);
-    w = std::max(w, plan_gemm(M, C, 4 * C, 1).ws_elems);
-    w = std::max(w, plan_gemm(M, m->V, C, 1).ws_elems);  // lm_head
-    return w;
-}
+// Split-K workspace of a step on `rows` rows of each of `batch` sequences.
+size_t gemm_ws_for(const fmlh_nanollm* m, int batch, int rows) { return engine_workspace_elems(m->C, m->V, batch, rows); }
 
 int ensure_ws(fmlh_nanollm* m, size_t elems) {
     if (elems <= m->ws_elems) return FMLH_OK;
@@ -1478,7 +1469,7 @@ int decode_steps(fmlh_nanollm* m, uint32_t n_steps, bool capture) {
         m->persist = false;
     }
     const int which = capture ? 1 : 0;
-    FMLH_TRY(ensure_ws(m, gemm_ws_for(m, (int)m->batch)));
+    FMLH_TRY(ensure_ws(m, gemm_ws_for(m, (int)m->batch, 1)));
     if (m->use_graph) {
         FMLH_TRY(build_graph(m, which));
         for (uint32_t i = 0; i < n_steps; ++i) FMLH_HIP(hipGraphLaunch(m->graph[which], stream()));
@@ -1519,7 +1510,7 @@ int do_prefill(fmlh_nanollm* m, const int32_t* prompts, uint32_t batch, uint32_t
         const int nb = (int)batch * (i + 1) / parts - (int)batch * i / parts;
         part_ws = std::max(part_ws, fused_part_ws(m, nb * (int)P, M));
     }
-    FMLH_TRY(ensure_ws(m, std::max(gemm_ws_for(m, M), (size_t)parts * part_ws)));
+    FMLH_TRY(ensure_ws(m, std::max(gemm_ws_for(m, (int)batch, (int)P), (size_t)parts * part_ws)));
     const size_t n = (size_t)M * m->C;
     hipLaunchKernelGGL(embed_kernel, dim3(blocks_for(n, 256, 8192u)), dim3(256), 0, s, m->x, m->hist,
                        m->HS, (int)P, 0, nullptr, m->tok, m->pos, m->C, M);
@@ -1651,7 +1642,7 @@ int fmlh_nanollm_create(const fmlh_nanollm_config* cfg, const fmlh_nanollm_weigh
         const hipError_t e = hipMemset(m->attn_ws, 0, aws * sizeof(float));
         if (e != hipSuccess) return fail(hip_fail(e, "hipMemset(attn_ws)", __FILE__, __LINE__));
     }
-    if ((rc = ensure_ws(m, gemm_ws_for(m, (int)B)))) return fail(rc);
+    if ((rc = ensure_ws(m, gemm_ws_for(m, (int)B, 1)))) return fail(rc);
     if ((rc = setup_persistent(m))) return fail(rc);
     if ((rc = setup_grouped(m))) return fail(rc);
     if ((rc = setup_relay(m))) return fail(rc);
@@ -1851,7 +1842,7 @@ int fmlh_nanollm_profile_op(fmlh_nanollm* m, int op, uint32_t iters, float* avg_
     const LayerW& w = m->layers[0];
     float* kc = m->kc;
     float* vc = m->vc;
-    FMLH_TRY(ensure_ws(m, gemm_ws_for(m, B)));
+    FMLH_TRY(ensure_ws(m, gemm_ws_for(m, B, 1)));
     // Position of the next decode step: the attention op reads keys 0..pos.
     const double keys = (double)m->prompt_len + m->generated - 1 + 1;
     // The kernels a decode step runs for the op: on the fused path (batched decode) the residual

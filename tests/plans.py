@@ -1,0 +1,21 @@
+"""The library's product plans, as host code computes them (no device needed; fmlh_internal_*)."""
+import collections
+import ctypes
+
+import freeml_amd as fh
+
+SKINNY_NN, SKINNY_NT, MFMA, SPLIT = range(4)  # GemmPlan::Kind
+Plan = collections.namedtuple("Plan", "kind tile k_groups splits ws_elems")
+
+
+def plan(M, N, K, b_trans):
+    out = [ctypes.c_int() for _ in range(4)]
+    ws = ctypes.c_size_t()
+    fh.lib().fmlh_internal_plan(M, N, K, b_trans, *map(ctypes.byref, out), ctypes.byref(ws))
+    return Plan(*(v.value for v in out), ws.value)
+
+
+def engine_workspace(C, V, batch, rows):
+    f = fh.lib().fmlh_internal_engine_workspace
+    f.restype = ctypes.c_size_t
+    return f(C, V, batch, rows)

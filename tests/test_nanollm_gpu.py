@@ -1013,6 +1013,25 @@ def test_fused_prefill_part_workspace(C, H, B, P, parts):
     om.close()
 
 
+def test_prefill_workspace_covers_the_head():
+    """50 of at most 64 sequences, 2 rows each: their lm_head plans more K-range partials than the
+    lm_head of 64 rows (engine creation) or any product of 100 rows (the blocks)."""
+    V, B, P = 8192, 50, 2
+    w = synth.make_weights(synth.NanoLLMShape(V, 16, 768, 12, 1), 31)
+    prompts = np.stack([synth.prompt_tokens(V, P, 900 + b) for b in range(B)])
+    m = fh.NanoLLM(w, max_batch=64)
+    try:
+        toks, logits = m.generate(prompts, 2, with_logits=True)
+    finally:
+        m.close()
+    om = oracle.OracleModel(w, nthreads=min(16, os.cpu_count() or 1))
+    for b in (0, 24, 49):
+        t_ref, l_ref = om.greedy(prompts[b], 2, cached=True)
+        assert rel_err_rows(logits[b], l_ref).max() <= REL_TOL, f"sequence {b}"
+        np.testing.assert_array_equal(toks[b], t_ref, err_msg=f"sequence {b}")
+    om.close()
+
+
 WIDE_CASES = [
     # (vocab, block, n_embed, n_head, layers, batch, prompt, steps)
     (65, 320, 256, 4, 2, 1, 40, 24),
