@@ -176,8 +176,10 @@ struct GemmPlan {
     int splits = 1, k_per_split = 0;
     size_t ws_elems = 0;
 };
-// one_range: without splitting K (kEpiKV writes its results as they are).
-GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false, size_t ws_max = kSplitWsFloats);
+// one_range: without splitting K (kEpiKV writes its results as they are).  split_takes: whether the
+// operands' strides allow the split tiles (gemm_split_takes).
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range = false, size_t ws_max = kSplitWsFloats,
+                   bool split_takes = true);
 
 // Split-K workspace of an engine step on `rows` rows of each of `batch` sequences: the blocks'
 // products on all of them, the lm_head's on the sequences' last rows.  (Fewer rows can plan more K

@@ -889,7 +889,7 @@ static int plan_cus() { return cu_count() > 0 ? cu_count() : 256; }
 // at least four K blocks.
 static int split_k_groups(float work_groups, int k) { return work_groups <= (float)plan_cus() && k >= 128 ? 2 : 1; }
 
-GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_max) {
+GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_max, bool split_takes) {
     GemmPlan p;
     if (M <= SK_MAXM) {
         if (b_trans) {
@@ -911,7 +911,7 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_m
     // to K 384 (256 x 384 x 384 9.3 / 9.7; 150 x 1024 x 256 8.6 / 8.1), and tiles times K to 4096
     // (1000 x 256 x 64 4.6 / 5.3).
     const bool small = (tiles64 <= 36 && K <= (b_trans ? 768 : 384)) || tiles64 * K <= 4096;
-    if ((M > 64 && !small) || (b_trans && 2 * tiles64 >= cus)) {
+    if (split_takes && ((M > 64 && !small) || (b_trans && 2 * tiles64 >= cus))) {
         p.kind = GemmPlan::kSplit;
         // Tile and K ranges by the time (us) they take, fitted on MI355X to 266 shapes (256 .. 14336
         // rows of 384 .. 1024-wide blocks, K to 50304) x 2 layouts x up to 15 choices: 0.5 % behind the
@@ -984,9 +984,11 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_m
 }
 
 namespace {
-// The plan of a call: that of plan_rows rows where given, with room for the call's own.
+// The plan of a call: that of plan_rows rows where given, with room for the call's own.  Row strides
+// beyond the split tiles' 32-bit offsets stay on the fp32 MFMA tiles.
 GemmPlan plan_for(const GemmArgs& g) {
-    GemmPlan p = plan_gemm(std::max(g.M, g.plan_rows), g.N, g.K, g.b_trans, g.epi == kEpiKV, g.ws_max);
+    GemmPlan p = plan_gemm(std::max(g.M, g.plan_rows), g.N, g.K, g.b_trans, g.epi == kEpiKV, g.ws_max,
+                           gemm_split_takes(split_args(g, 64)));
     if (g.plan_rows > g.M && p.splits > 1) p.ws_elems = (size_t)p.splits * g.M * g.N;
     return p;
 }
@@ -1289,9 +1291,11 @@ float* noalloc_scratch() {
 
 // ---- plans, for tests (no device needed) ----------------------------------------------------
 
-extern "C" int fmlh_internal_plan(int M, int N, int K, int b_trans, int* kind, int* tile, int* k_groups, int* splits,
-                                  size_t* ws_elems) {
-    const GemmPlan p = plan_gemm(M, N, K, b_trans);
+extern "C" int fmlh_internal_plan(int M, int N, int K, int b_trans, int lda, int ldb, int* kind, int* tile, int* k_groups,
+                                  int* splits, size_t* ws_elems) {
+    GemmArgs g;
+    g.M = M; g.N = N; g.K = K; g.b_trans = b_trans; g.lda = lda; g.ldb = ldb;
+    const GemmPlan p = plan_for(g);
     *kind = p.kind; *tile = p.bm; *k_groups = p.k_groups; *splits = p.splits; *ws_elems = p.ws_elems;
     return FMLH_OK;
 }

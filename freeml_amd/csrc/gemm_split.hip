@@ -465,7 +465,8 @@ bool gemm_split_takes(const SplitGemm& g) {
 }
 
 int gemm_split(const SplitGemm& g) {
-    FMLH_REQUIRE(gemm_split_takes(g), "gemm_split: %dx%dx%d operands not aligned", g.M, g.N, g.K);
+    FMLH_REQUIRE(gemm_split_takes(g), "gemm_split: %dx%dx%d, row strides %d and %d: not aligned or too long", g.M, g.N, g.K,
+                 g.lda, g.ldb);
     FMLH_REQUIRE(g.splits == 1 || (g.partial && g.k_per_split % 16 == 0), "gemm_split: split K without room");
     if (g.tile == 128) return by_layout<128, 128, 16, 1>(g);
     return g.k_groups == 2 ? by_layout<64, 64, 32, 2>(g) : by_layout<64, 64, 32, 1>(g);

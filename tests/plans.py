@@ -8,10 +8,11 @@ SKINNY_NN, SKINNY_NT, MFMA, SPLIT = range(4)  # GemmPlan::Kind
 Plan = collections.namedtuple("Plan", "kind tile k_groups splits ws_elems")
 
 
-def plan(M, N, K, b_trans):
+def plan(M, N, K, b_trans, lda=None, ldb=None):
+    """Plan of a product of 16-byte aligned operands (row strides: those of packed matrices)."""
     out = [ctypes.c_int() for _ in range(4)]
     ws = ctypes.c_size_t()
-    fh.lib().fmlh_internal_plan(M, N, K, b_trans, *map(ctypes.byref, out), ctypes.byref(ws))
+    fh.lib().fmlh_internal_plan(M, N, K, b_trans, lda or K, ldb or (K if b_trans else N), *map(ctypes.byref, out), ctypes.byref(ws))
     return Plan(*(v.value for v in out), ws.value)
 
 

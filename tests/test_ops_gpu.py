@@ -193,6 +193,37 @@ def test_mul_many_k_ranges(shape, mode):
     assert np.all(np.abs(dC.numpy() - A64 @ W64) <= (0.75 * K + 24) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
 
 
+# Row strides of 2^22 floats and more: past the split tiles' 32-bit offsets, on the fp32 tiles.
+@pytest.mark.parametrize("M,N,K,bt,lda,ldb", [(1000, 1000, 32, 0, 32, 1 << 22), (130, 4096, 32, 0, 1 << 22, 4096),
+                                              (130, 4096, 32, 1, (1 << 22) + 4, 32), (4096, 130, 32, 1, 32, 1 << 22)])
+@pytest.mark.parametrize("epi", [fh.EPI_NONE, fh.EPI_RESID])
+def test_gemm_ex_long_row_strides(M, N, K, bt, lda, ldb, epi):
+    print(f"gemm_ex M={M} N={N} K={K} bt={bt} lda={lda} ldb={ldb} epi={epi}", flush=True)
+    r = _rng(M + N)
+    A, W = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    Rm = r.standard_normal((M, N)).astype(np.float32)
+
+    def rows(X, ld):
+        d = fh.DeviceArray(X.shape[0] * ld)
+        for i, row in enumerate(np.ascontiguousarray(X)):
+            fh.call("fmlh_memcpy_h2d", d.at(i * ld), row.ctypes.data, row.nbytes)
+        return d
+
+    dA, dW, dC = rows(A, lda), rows(W.T if bt else W, ldb), D(Rm)
+    fh.gemm_ex(dA.ptr, lda, dW.ptr, ldb, bt, dC.ptr, N, M, N, K, epi, dC.ptr if epi == fh.EPI_RESID else 0, N)
+    _close(dC.numpy(), A.astype(np.float64) @ W + (Rm if epi == fh.EPI_RESID else 0), 1e-5)
+
+
+def test_mul_4m_columns():
+    M, N, K = 65, 1 << 22, 16
+    r = _rng(9)
+    A, W = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N), dtype=np.float32)
+    dA, dW, dC = D(A), D(W), fh.DeviceArray((M, N))
+    fh.mul(fh.NONE, dC.ptr, dA.ptr, dW.ptr, M, N, K)
+    got, cols = dC.numpy(), np.r_[0:200, r.integers(0, N, 2000), N - 200:N]
+    _close(got[:, cols], A.astype(np.float64) @ W[:, cols], 1e-5)
+
+
 # Strided products of 64 tiles' worth of outputs and more (the split bf16 tiles): every mode, both
 # index orders of each operand (rows or columns contiguous), batched planes, K with a remainder,
 # row strides that keep 16-byte rows and ones that do not (the wave-split kernel), 128-wide tiles.

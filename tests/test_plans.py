@@ -1,7 +1,7 @@
 """Plans of the products, on the host (256 CUs where there is no device)."""
 import random
 
-from plans import engine_workspace, plan
+from plans import MFMA, SPLIT, engine_workspace, plan
 
 
 def test_engine_workspace_holds_every_product_of_a_prefill():
@@ -15,3 +15,12 @@ def test_engine_workspace_holds_every_product_of_a_prefill():
         room, M = engine_workspace(C, V, batch, P), batch * P
         for rows, N, K in ((M, 3 * C, C), (M, C, C), (M, 4 * C, C), (M, C, 4 * C), (batch, V, C)):
             assert plan(rows, N, K, 1).ws_elems <= room, (C, V, batch, P, rows, N, K)
+
+
+def test_row_strides_beyond_32_bit_offsets_stay_on_fp32_tiles():
+    far = 1 << 22
+    assert plan(1000, 1000, 32, 0, ldb=far - 4).kind == SPLIT and plan(1000, 1000, 32, 0, ldb=far).kind == MFMA
+    for bt in (0, 1):
+        assert plan(130, 4096, 32, bt).kind == SPLIT and plan(130, 4096, 32, bt, lda=far).kind == MFMA
+    assert plan(4096, 130, 32, 1, ldb=far).kind == MFMA
+    assert plan(65, far, 16, 0).kind == MFMA and plan(65, 64, far, 0).kind == MFMA and plan(65, 64, far, 1).kind == MFMA
