@@ -308,7 +308,8 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
         __syncthreads();
     }
     // What the split cannot carry -- infinities (and values that round to one in bf16), which
-    // leave a NaN in the sums, and rows of tiny elements -- is multiplied again in fp32.
+    // leave a NaN in the sums, products whose rounded-up parts pass fp32's range though the product
+    // does not, which leave an infinity, and rows of tiny elements -- is multiplied again in fp32.
     {
         uint32_t* rmax = reinterpret_cast<uint32_t*>(all_lds);  // free since the last barrier
         for (int i = threadIdx.x; i < BM + BN; i += KG * NT) rmax[i] = 0u;
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
 #pragma unroll
             for (int j = 0; j < NBK; ++j)
 #pragma unroll
-                for (int r = 0; r < AR; ++r) redo |= acc[i][j][r] != acc[i][j][r];
+                for (int r = 0; r < AR; ++r) redo |= !(fabsf(acc[i][j][r]) < INFINITY);
         if (__syncthreads_or(redo)) {
             clear();
             for (int k = kbeg_wg; k < kend_wg; k += 64 / MT) {

@@ -10,6 +10,7 @@ import pytest
 
 import freeml_amd as fh
 import oracle
+from plans import SPLIT, plan
 
 pytestmark = pytest.mark.gpu
 
@@ -176,6 +177,44 @@ def test_gemm_split_bf16_special_values(tile, monkeypatch):
     # sums below fp32's smallest normal number (1e-34 * 1e-33) are not held to a relative bound
     err = np.abs(got - ref)[fin]
     assert np.all(err <= (0.75 * K + 8) * 2.0 ** -24 * prod[fin] + 2.0 ** -126)
+
+
+# Launches of the split tiles: 64 x 64 with one and with two groups of waves, K ranges, 128 x 128.
+SPLIT_LAUNCHES = [((1100, 900, 64), "", (64, 1, 1)), ((700, 600, 400), "", (64, 2, 1)), ((300, 260, 1600), "", (64, 2, 10)),
+                  ((700, 600, 400), "128x128", (128, 1, 1))]
+
+
+def _split_launch(shape, tile, launch, bt, monkeypatch):
+    """Checks that a product takes the split tiles as meant, whatever the planner has become."""
+    if tile:
+        monkeypatch.setenv("FMLH_GEMM_NT_TILE", tile)
+    p = plan(*shape, bt)
+    assert p.kind == SPLIT and (p.tile, p.k_groups, p.splits) == launch, p
+
+
+def _gemm_ex(A, W, bt):
+    (M, K), N = A.shape, W.shape[1]
+    dA, dW, dC = D(A), D(np.ascontiguousarray(W.T) if bt else W), fh.DeviceArray((M, N))
+    fh.gemm_ex(dA.ptr, K, dW.ptr, K if bt else N, bt, dC.ptr, N, M, N, K, fh.EPI_NONE, 0, N)
+    return dC.numpy().astype(np.float64)
+
+
+# Sums within 2^-8 of fp32's largest number: a0 b0 alone is past it where both bf16 parts are rounded
+# up.  One such element per row of A, its partner in B, everything else small.
+@pytest.mark.parametrize("bt", [0, 1])
+@pytest.mark.parametrize("shape,tile,launch", SPLIT_LAUNCHES)
+def test_gemm_split_near_the_largest_number(shape, tile, launch, bt, monkeypatch):
+    print(f"near the largest number {shape} {tile} bt={bt}", flush=True)
+    _split_launch(shape, tile, launch, bt, monkeypatch)
+    M, N, K = shape
+    r = _rng(K)
+    A, W = (r.standard_normal((M, K)) * 1e-3).astype(np.float32), (r.standard_normal((K, N)) * 1e-3).astype(np.float32)
+    A[:, 5], W[5, :] = 0.0, 0.0
+    A[::3, 5] = W[5, ::2] = np.float32(1.998 * 2.0 ** 63)  # bf16: 2^64
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    ref = A64 @ W64
+    assert 0.99 * 2.0 ** 128 < np.abs(ref).max() < np.finfo(np.float32).max
+    assert np.all(np.abs(_gemm_ex(A, W, bt) - ref) <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
 
 
 # Many K ranges (up to 16, the last one short or ragged) and partials beyond the no-alloc array
