@@ -18,11 +18,11 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{x, y}, bf16x2));
 }
 
-// Eight floats -> their three bf16 planes (one 16-byte unit each).
-__device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&p)[3]) {
+// Eight floats, times `scale`, -> their three bf16 planes (one 16-byte unit each).
+__device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&p)[3], float scale = 1.0f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float x = v[2 * i], y = v[2 * i + 1];
+        const float x = v[2 * i] * scale, y = v[2 * i + 1] * scale;
         const uint32_t p0 = pack_bf16(x, y);
         const float rx = x - __uint_as_float(p0 << 16), ry = y - __uint_as_float(p0 & 0xffff0000u);
         const uint32_t p1 = pack_bf16(rx, ry);

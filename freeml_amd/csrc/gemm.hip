@@ -1124,7 +1124,7 @@ bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M,
     q->A = L; q->a_kc = a_k == 1; q->lda = (int)std::min<uint32_t>(a_k == 1 ? a_r : a_k, INT32_MAX); q->a_plane = l_plane;
     q->B = R; q->b_kc = b_k == 1; q->ldb = (int)std::min<uint32_t>(b_k == 1 ? b_r : b_k, INT32_MAX); q->b_plane = r_plane;
     q->M = (int)M; q->N = (int)N; q->K = (int)K; q->planes = (int)batch;
-    q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * cu_count() ? 128 : 64;
+    q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * plan_cus() ? 128 : 64;
     if (q->tile == 64) q->k_groups = split_k_groups((float)((M + 63) / 64) * ((N + 63) / 64) * batch, (int)K);
     return gemm_split_takes(*q);
 }
@@ -1298,6 +1298,16 @@ extern "C" int fmlh_internal_plan(int M, int N, int K, int b_trans, int lda, int
     const GemmPlan p = plan_for(g);
     *kind = p.kind; *tile = p.bm; *k_groups = p.k_groups; *splits = p.splits; *ws_elems = p.ws_elems;
     return FMLH_OK;
+}
+
+extern "C" int fmlh_internal_strided_tile(int mode, uint32_t M, uint32_t N, uint32_t K, uint32_t l_rs, uint32_t l_cs,
+                                          uint32_t r_rs, uint32_t r_cs, uint32_t o_rs, uint32_t o_cs, uint32_t batch,
+                                          size_t l_plane, size_t r_plane) {
+    SplitGemm q;
+    const bool tl = mode == FMLH_TRANSPOSE_LEFT || mode == FMLH_TRANSPOSE_BOTH;
+    const bool tr = mode == FMLH_TRANSPOSE_RIGHT || mode == FMLH_TRANSPOSE_BOTH;
+    return strided_split(tl, tr, nullptr, nullptr, M, N, K, l_rs, l_cs, r_rs, r_cs, o_rs, o_cs, batch, l_plane, r_plane, &q)
+               ? q.tile : 0;
 }
 
 extern "C" size_t fmlh_internal_engine_workspace(int C, int V, int batch, int rows) {

@@ -22,7 +22,7 @@
 // The operands are split while they are staged (registers -> LDS), so fp32 matrices of any
 // layout are read once and nothing is kept.  Per 128 x 128 x 16 block a work-group's matrix cores
 // need ~770 clocks, its LDS ~580 (three planes written once, read by two waves) and its
-// vector units ~500 (5.5 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
+// vector units ~540 (6 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
 // every plane of half as many products) and serve the products with too few large tiles.  The
 // launch bounds matter: left alone, the compiler takes 267 registers for the large tile (one wave
 // per SIMD: 4096 x 3072 x 768 125 us instead of 107).
@@ -38,9 +38,14 @@ namespace {
 
 __device__ __forceinline__ float gelu_ref(float x) { return 0.5f * x * (1.0f + erff(x / 1.41421354f)); }
 
-// Rows whose largest element is below this (and not zero) do not split exactly any more: the
-// third part falls under bf16's smallest normal.
-constexpr float kSplitTiny = 0x1p-90f;
+// Elements are staged times 2^24 and sums taken back by 2^-48, both exact.  The MFMAs take bf16 numbers
+// below 2^-126 as zero (measured; their fp32 sums keep subnormal bits), so unscaled, an element below
+// 2^-102 lost its last parts, which showed where it met the only large partner of its row.  Scaled,
+// the parts of every fp32 number, subnormal ones included, are zero or normal.  Elements from
+// 2^104 and sums from 2^80 on leave the range at its upper end instead and are multiplied again in
+// fp32.  The multiplication costs 1 % (dense layers of a 768-wide block on 2500 rows 266 -> 270 us); flagging
+// tiny elements instead, and testing sums against them, cost 2 to 3.5.
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
 
 // The MFMAs of the two tile sizes.  Lane l of an MT x MT product supplies row / column l % MT and
 // the 8 consecutive k of octet l / MT; accumulator register r holds row 8 (r / 4) + 4 (l / MT) +
@@ -142,12 +147,6 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
     const float* a_base = A + (AKC ? (size_t)row0 * lda : (size_t)row0);
     const float* b_base = B + (BKC ? (size_t)col0 * ldb : (size_t)col0);
     float va[NA][8], vb[NB][8];
-    float amax[NA], bmax[NB];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) amax[i] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NB; ++i) bmax[i] = 0.0f;
-
     auto load_unit = [&](float (&v)[8], const float* base, uint32_t off, bool kc, int ld, int kk, bool full) {
         const char* p = reinterpret_cast<const char*>(base) + off;
         if (kc) {
@@ -183,18 +182,14 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             uintx4 p[3];
-            split8(va[i], p);
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) amax[i] = fmaxf(fmaxf(amax[i], fabsf(va[i][e])), fabsf(va[i][e + 1]));
+            split8(va[i], p, kSplitScale);
 #pragma unroll
             for (int q = 0; q < 3; ++q) sa[(q * BM + a_row[i]) * U + (a_oct[i] ^ swz(a_row[i]))] = p[q];
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             uintx4 p[3];
-            split8(vb[i], p);
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) bmax[i] = fmaxf(fmaxf(bmax[i], fabsf(vb[i][e])), fabsf(vb[i][e + 1]));
+            split8(vb[i], p, kSplitScale);
 #pragma unroll
             for (int q = 0; q < 3; ++q) sb[(q * BN + b_row[i]) * U + (b_oct[i] ^ swz(b_row[i]))] = p[q];
         }
@@ -307,23 +302,10 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
         }
         __syncthreads();
     }
-    // What the split cannot carry -- infinities (and values that round to one in bf16), which
-    // leave a NaN in the sums, products whose rounded-up parts pass fp32's range though the product
-    // does not, which leave an infinity, and rows of tiny elements -- is multiplied again in fp32.
+    // What leaves the range is multiplied again in fp32: infinities and elements that scaled or rounded
+    // to bf16 become one, which leave a NaN in the sums, and sums past the scaled range.
     {
-        uint32_t* rmax = reinterpret_cast<uint32_t*>(all_lds);  // free since the last barrier
-        for (int i = threadIdx.x; i < BM + BN; i += KG * NT) rmax[i] = 0u;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < NA; ++i) atomicMax(&rmax[a_row[i]], __float_as_uint(amax[i]));
-#pragma unroll
-        for (int i = 0; i < NB; ++i) atomicMax(&rmax[BM + b_row[i]], __float_as_uint(bmax[i]));
-        __syncthreads();
         bool redo = false;
-        for (int i = threadIdx.x; i < BM + BN; i += KG * NT) {
-            const float v = __uint_as_float(rmax[i]);
-            redo |= v > 0.0f && v < kSplitTiny;
-        }
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -352,6 +334,13 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
                     for (int j = 0; j < NBK; ++j)
                         acc[i][j] = Mfma<MT>::fp32(av[i], bv[j], acc[i][j]);
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NBK; ++j)
+#pragma unroll
+                    for (int r = 0; r < AR; ++r) acc[i][j][r] *= kSplitUnscale;
         }
     }
 

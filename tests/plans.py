@@ -20,3 +20,10 @@ def engine_workspace(C, V, batch, rows):
     f = fh.lib().fmlh_internal_engine_workspace
     f.restype = ctypes.c_size_t
     return f(C, V, batch, rows)
+
+
+def strided_tile(mode, M, N, K, l_rs, l_cs, r_rs, r_cs, o_rs, o_cs, batch=1, l_plane=0, r_plane=0):
+    """Side of the split tiles a strided product of 16-byte aligned operands takes; 0: none."""
+    u, z = ctypes.c_uint32, ctypes.c_size_t
+    return fh.lib().fmlh_internal_strided_tile(mode, *map(u, (M, N, K, l_rs, l_cs, r_rs, r_cs, o_rs, o_cs, batch)),
+                                               z(l_plane), z(r_plane))

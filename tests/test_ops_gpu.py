@@ -10,7 +10,7 @@ import pytest
 
 import freeml_amd as fh
 import oracle
-from plans import SPLIT, plan
+from plans import SPLIT, plan, strided_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -215,6 +215,46 @@ def test_gemm_split_near_the_largest_number(shape, tile, launch, bt, monkeypatch
     ref = A64 @ W64
     assert 0.99 * 2.0 ** 128 < np.abs(ref).max() < np.finfo(np.float32).max
     assert np.all(np.abs(_gemm_ex(A, W, bt) - ref) <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
+
+
+# A tiny element (of A, of B, of both; down to fp32's subnormals) in rows of normal ones, where it
+# meets a large partner and the other elements meet zeros: as accurate as anywhere else.  Every other
+# column has normal partners beside the tiny ones.
+@pytest.mark.parametrize("bt", [0, 1])
+@pytest.mark.parametrize("shape,tile,launch", SPLIT_LAUNCHES)
+def test_gemm_split_tiny_elements_beside_normal_ones(shape, tile, launch, bt, monkeypatch):
+    _split_launch(shape, tile, launch, bt, monkeypatch)
+    M, N, K = shape
+    for t in (-98, -103, -110, -118, -126, -140):
+        print(f"tiny elements 2^{t} {shape} {tile} bt={bt}", flush=True)
+        r = _rng(K - t)
+        A, W = r.standard_normal((M, K)), r.standard_normal((K, N))
+        A[::2, 7] *= 2.0 ** t
+        W[:, ::2] = 0
+        W[7, ::2] = r.standard_normal((N + 1) // 2) * 2.0 ** 60
+        A[5::32, :] = 0
+        A[5::32, 9] = r.standard_normal(len(range(5, M, 32))) * 2.0 ** 40
+        W[9, 1::32] *= 2.0 ** t
+        A, W = A.astype(np.float32), W.astype(np.float32)
+        A64, W64 = A.astype(np.float64), W.astype(np.float64)
+        err, prod = np.abs(_gemm_ex(A, W, bt) - A64 @ W64), np.abs(A64) @ np.abs(W64)
+        # (2^-149: sums that are subnormal themselves)
+        assert np.all(err <= (0.75 * K + 8) * (2.0 ** -24 * prod + 2.0 ** -149)), t
+
+
+def test_matmul_strided_split_tiny_elements_beside_normal_ones():
+    M, N, K = 600, 500, 130
+    assert strided_tile(fh.LEFT, M, N, K, M, 1, N, 1, N, 1) == 64
+    r = _rng(2)
+    A, W = r.standard_normal((M, K)), r.standard_normal((K, N))
+    A[:, 7] *= 2.0 ** -120
+    W[:, ::2] = 0
+    W[7, ::2] = 2.0 ** 60
+    A, W = A.astype(np.float32), W.astype(np.float32)
+    dA, dW, dC = D(np.ascontiguousarray(A.T)), D(W), fh.DeviceArray((M, N))
+    fh.matmul_strided(fh.LEFT, dC.ptr, dA.ptr, dW.ptr, M, N, K, M, 1, N, 1, N, 1)
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    assert np.all(np.abs(dC.numpy() - A64 @ W64) <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
 
 
 # Many K ranges (up to 16, the last one short or ragged) and partials beyond the no-alloc array
