@@ -566,11 +566,17 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(
 //     16-byte units of 8 consecutive dims of a key, and of 8 keys (in the order above) of a dim.
 //     Unit o of row r lies at o ^ (r % 8): any 8 consecutive lanes on one row each, or on one
 //     row's 8 units, touch distinct banks.
-// Infinite keys or values give NaN (their parts are infinity minus infinity), where the products
-// alone would keep some infinities; the LayerNorm behind either makes NaN of both.
+//   * bf16 numbers end at 2^-133, so of an element below 2^-110 up to 2^-134 goes missing.  Q is split times
+//     2^37 (nothing of it is lost then; the scores' factor takes it back): what is missing of a tiny K
+//     moves a score by 2^-37 at most while Q is below 2^91, and beyond that the scores leave fp32's range.
+//     What is missing of tiny P and V is below an fp32 rounding of a sum of at least 2^-110 per key and
+//     unit of the dim's largest value.  A wave with a smaller sum, or one that is infinite or NaN
+//     (infinite keys and values, parts that round past the range), does its 32 queries again on the
+//     fp32 MFMAs, K and V straight from memory.
 constexpr int kAttnQPerWave = 32;
 constexpr int kAttnQPerWG = 4 * kAttnQPerWave;
 constexpr int kAttnKT = 64;  // keys per tile
+constexpr float kAttnQScale = 0x1p37f, kAttnLost = 0x1p-110f;
 
 __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
     const float* __restrict__ qkv, int qkv_ld, const float* __restrict__ kc,
@@ -579,11 +585,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
     constexpr int HD = 64, U = 8;  // 16-byte units per row and plane
     __shared__ uintx4 kp[3][kAttnKT * U];  // [plane][key][unit]
     __shared__ uintx4 vp[3][HD * U];       // [plane][dim][unit]
+    __shared__ __attribute__((aligned(16))) uint32_t vmax_sh[HD];  // largest |V| of each dim (bits)
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, c = lane & 31;
+    if (tid < HD) vmax_sh[tid] = 0u;
     // Dispatched x-fastest: every (sequence, head) of a query block, longest blocks first.
     const int qb = gridDim.y - 1 - blockIdx.y;
     const int bh = blockIdx.x, b = bh / H, hh = bh % H;
@@ -597,6 +605,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
     // 16 (o / 2) + 4 (o % 2) + {0..3, 8..11} of octet o = u / 64.  Keys past the work-group's last
     // query read that query's row (finite values, masked out).
     float kv[2][8], vv[2][8];
+    float vmax = 0.f;  // of the thread's share of V: dim `lane` of its keys
     auto load = [&](int tile) {
         const int t0 = tile * kAttnKT;
 #pragma unroll
@@ -625,6 +634,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
             for (int q = 0; q < 3; ++q) kp[q][(u / 8) * U + ((u % 8) ^ (u / 8 & 7))] = p[q];
             split8(vv[i], p);
 #pragma unroll
+            for (int e = 0; e < 8; e += 2) vmax = fmaxf(fmaxf(vmax, fabsf(vv[i][e])), fabsf(vv[i][e + 1]));
+#pragma unroll
             for (int q = 0; q < 3; ++q) vp[q][(u % 64) * U + ((u / 64) ^ (u & 7))] = p[q];
         }
     };
@@ -633,28 +644,70 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
     // Q^T operand: lane (h, c) holds dims 16 s + 8 h .. + 7 of query q0 + c (rows past the
     // sequence read its last row; their results are not stored).
     const bool wave_live = q0 < rows_per_seq;
+    const float* q_row = qkv + ((size_t)b * rows_per_seq + min(q0 + c, rows_per_seq - 1)) * qkv_ld + hh * HD;
     bf16x8 qp[3][4];
     {
-        const int qrow = min(q0 + c, rows_per_seq - 1);
-        const float* qr = qkv + ((size_t)b * rows_per_seq + qrow) * qkv_ld + hh * HD + 8 * h;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const floatx4 lo = *reinterpret_cast<const floatx4*>(qr + 16 * s);
-            const floatx4 hi = *reinterpret_cast<const floatx4*>(qr + 16 * s + 4);
+            const floatx4 lo = *reinterpret_cast<const floatx4*>(q_row + 16 * s + 8 * h);
+            const floatx4 hi = *reinterpret_cast<const floatx4*>(q_row + 16 * s + 8 * h + 4);
             const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             uintx4 p[3];
-            split8(v, p);
+            split8(v, p, kAttnQScale);
 #pragma unroll
             for (int q = 0; q < 3; ++q) qp[q][s] = __builtin_bit_cast(bf16x8, p[q]);
         }
     }
     floatx16 o[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-    float mrun = -INFINITY, lsum = 0.f;
+    float mrun, lsum;
     const int qpos = q0 + c;
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+        mrun = -INFINITY;
+        lsum = 0.f;
+    };
+    // Online softmax for query c over this lane's 32 keys of the tile at t0 and the partner half's:
+    // scores times `factor` -> probabilities.
+    auto softmax = [&](floatx16 (&s)[2], int t0, float factor) {
+        const bool diag = t0 + kAttnKT - 1 > q0;  // some key of the tile follows some query
+        float mt = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float v = s[j][r] * factor;
+                if (diag) {
+                    const int kpos = t0 + 32 * j + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (kpos > qpos) v = -INFINITY;
+                }
+                s[j][r] = v;
+                mt = fmaxf(mt, v);
+            }
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        const float mnew = fmaxf(mrun, mt);  // finite: tile 0 holds key 0 <= every query
+        const float corr = exp2f(mrun - mnew);
+        mrun = mnew;
+        float ls = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = exp2f(s[j][r] - mnew);
+                s[j][r] = p;
+                ls += p;
+            }
+        lsum = lsum * corr + ls;
+        if (__ballot(corr != 1.0f)) {  // some query's running max moved
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[i][r] *= corr;
+        }
+    };
+    clear();
 
     for (int tile = 0; tile < ntiles; ++tile) {
         // Every wave has read the tile before; the requested loads stay in flight over a barrier.
@@ -689,41 +742,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
                     s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[kSplitA[q]][j], qp[kSplitB[q]][st], s[j], 0, 0, 0);
         }
 
-        // Online softmax for query c over this lane's 32 keys and the partner half's.
-        const bool diag = t0 + kAttnKT - 1 > q0;  // some key of the tile follows some query
-        float mt = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float v = s[j][r] * scale_log2;
-                if (diag) {
-                    const int kpos = t0 + 32 * j + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (kpos > qpos) v = -INFINITY;
-                }
-                s[j][r] = v;
-                mt = fmaxf(mt, v);
-            }
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mnew = fmaxf(mrun, mt);  // finite: tile 0 holds key 0 <= every query
-        const float corr = exp2f(mrun - mnew);
-        mrun = mnew;
-        float ls = 0.f;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = exp2f(s[j][r] - mnew);
-                s[j][r] = p;
-                ls += p;
-            }
-        lsum = lsum * corr + ls;
-        if (__ballot(corr != 1.0f)) {  // some query's running max moved
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[i][r] *= corr;
-        }
+        softmax(s, t0, scale_log2 / kAttnQScale);
 
         // O^T += V^T P^T; row rho of O^T block i is dim 32 i + rho.
 #pragma unroll
@@ -751,11 +770,58 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
                             va[kSplitA[q]][i], __builtin_bit_cast(bf16x8, pp[kSplitB[q]]), o[i], 0, 0, 0);
             }
     }
+    atomicMax(&vmax_sh[lane], __float_as_uint(vmax));
+    __syncthreads();
     if (!wave_live) return;
+    // Register r of block i: dim 32 i + 8 (r / 4) + 4 h + r % 4.
+    bool redo = false;
+    const float lost = kAttnLost * (last_q + 1);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uintx4 vm = *reinterpret_cast<const uintx4*>(&vmax_sh[32 * i + 8 * u + 4 * h]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = fabsf(o[i][4 * u + e]);
+                redo |= !(a < INFINITY) || (vm[e] != 0u && a < lost * fmaxf(__uint_as_float(vm[e]), 1.0f));
+            }
+        }
+    if (__ballot(redo)) {
+        clear();
+#pragma unroll 1
+        for (int t0 = 0; t0 <= min(q0 + kAttnQPerWave - 1, last_q); t0 += kAttnKT) {
+            floatx16 s[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
+#pragma unroll 1
+            for (int u = 0; u < 32; u += 4) {  // k-step: dim u + e of either half of them
+                const int d = 32 * h + u;
+                const floatx4 qv = *reinterpret_cast<const floatx4*>(q_row + d);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const floatx4 ka =
+                        *reinterpret_cast<const floatx4*>(kbase + (size_t)min(t0 + 32 * j + c, last_q) * HD + d);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[e], qv[e], s[j], 0, 0, 0);
+                }
+            }
+            softmax(s, t0, scale_log2);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {  // k-step: the key register r of block j holds in either half
+                    const float* vr = vbase + (size_t)min(t0 + 32 * j + 8 * (r >> 2) + 4 * h + (r & 3), last_q) * HD + c;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[32 * i], s[j][r], o[i], 0, 0, 0);
+                }
+        }
+    }
     const float inv = 1.0f / (lsum + __shfl_xor(lsum, 32));
     if (qpos < rows_per_seq) {
         float* dst = y + ((size_t)b * rows_per_seq + qpos) * y_ld + hh * HD;
-        // Register r of block i: dim 32 i + 8 (r / 4) + 4 h + r % 4.
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll

@@ -38,9 +38,9 @@ namespace {
 
 __device__ __forceinline__ float gelu_ref(float x) { return 0.5f * x * (1.0f + erff(x / 1.41421354f)); }
 
-// Elements are staged times 2^24 and sums taken back by 2^-48, both exact.  The MFMAs take bf16 numbers
-// below 2^-126 as zero (measured; their fp32 sums keep subnormal bits), so unscaled, an element below
-// 2^-102 lost its last parts, which showed where it met the only large partner of its row.  Scaled,
+// Elements are staged times 2^24 and sums taken back by 2^-48, both exact.  bf16 numbers end at 2^-133
+// (the MFMAs take subnormal ones as they are: measured), so unscaled, the parts of an element below
+// 2^-110 no longer add up to it, which showed where it met the only large partner of its row.  Scaled,
 // the parts of every fp32 number, subnormal ones included, are zero or normal.  Elements from
 // 2^104 and sums from 2^80 on leave the range at its upper end instead and are multiplied again in
 // fp32.  The multiplication costs 1 % (dense layers of a 768-wide block on 2500 rows 266 -> 270 us); flagging

@@ -308,6 +308,99 @@ def test_prefill_attention_on_matrix_cores_matches_per_lane_kernel(kernel, name,
     assert rel_err_rows(fast, ref).max() <= 1e-5
 
 
+def _one_layer_float64(w, ids):
+    """Logits of every row of a one-layer model; keys rounded to fp32 (where they may overflow)."""
+    from scipy.special import erf
+
+    def f(a):
+        return np.asarray(a, np.float64)
+
+    def ln(x, g):
+        d = x - x.mean(-1, keepdims=True)
+        return d / np.sqrt((d * d).mean(-1, keepdims=True) + 1e-5) * f(g)
+
+    l, C, H = w.layers[0], w.shape.n_embed, w.shape.n_head
+    T, hd = len(ids), w.shape.n_embed // w.shape.n_head
+    x = f(w.tok_emb)[ids] + f(w.pos_emb)[:T]
+    with np.errstate(all="ignore"):
+        q, k, v = np.split(ln(x, l.ln0_g) @ f(l.w_qkv), 3, axis=1)
+        k = f(k.astype(np.float32))
+        y = np.empty((T, C))
+        for h in range(H):
+            c = slice(h * hd, (h + 1) * hd)
+            for i in range(T):
+                s = (k[:i + 1, c] * q[i, c]).sum(-1) / np.sqrt(hd)
+                p = np.exp(s - s.max())
+                y[i, c] = p @ v[:i + 1, c] / p.sum()
+        x = x + y @ f(l.w_proj).T
+        h4 = ln(x, l.ln1_g) @ f(l.w_fc)
+        x = x + 0.5 * h4 * (1 + erf(h4 / np.sqrt(2))) @ f(l.w_proj2)
+        return ln(x, w.lnf_g) @ f(w.lm_head).T
+
+
+@pytest.mark.parametrize("case", ["unit", "tiny_v", "some_dims_tiny", "tiny_k_large_q", "large_k_tiny_q",
+                                  "tiny_probabilities", "infinite_keys"])
+@pytest.mark.parametrize("T", [256, 300])
+def test_prefill_attention_over_the_range_of_fp32(case, T):
+    """Every row's logits of a one-layer model (head_dim 64, both heads) against float64, where Q, K, V or the
+    probabilities lie at the ends of fp32's range: on the bf16 parts and on the fp32 pass behind them."""
+    print(f"attention range {case} T={T}", flush=True)
+    C, V = 128, 65
+    w = synth.make_weights(synth.NanoLLMShape(V, T, C, 2, 1, tied=False), 77, std=0.1)
+    l = w.layers[0]
+    q, k, v = l.w_qkv[:, :C], l.w_qkv[:, C:2 * C], l.w_qkv[:, 2 * C:]  # views
+    ids = np.array(synth.prompt_tokens(V, T, 5))
+    if case == "tiny_v":  # and the projection brings them back
+        v *= np.float32(2.0 ** -122)
+        l.w_proj *= np.float32(2.0 ** 122)
+    elif case == "some_dims_tiny":
+        s = np.where(np.arange(C) % 3 == 0, 2.0 ** -122, 1.0).astype(np.float32)
+        v *= s
+        l.w_proj /= s
+    elif case in ("tiny_k_large_q", "large_k_tiny_q"):
+        e = np.float32(2.0 ** (120 if case == "tiny_k_large_q" else -120))
+        q *= e
+        k /= e
+    elif case == "tiny_probabilities":
+        # Tokens 2..: dims 0..63; tokens 0 and 1: dims 64..127.  Only tokens 0 and 1 have values, and every
+        # other token's query gives their keys some 2^-120 of the weight each.
+        w.pos_emb[:] = 0
+        sign = np.tile(np.float32([0.125, -0.125]), 32)  # (means of exactly zero)
+        w.tok_emb[:] = 0
+        w.tok_emb[2:, :64] = sign
+        w.tok_emb[0, 64:] = sign
+        w.tok_emb[1, 64:] = np.tile(np.float32([0.125, 0.125, -0.125, -0.125]), 16)
+        q[:], k[:], v[:64] = 0, 0, 0
+        for h in (0, 64):  # in one dim of each head, q and k of tokens 2..; k of 0 and 1 differ a little
+            q[0, h], k[0, h], k[65, h] = 1.0, 1.0, 0.01
+        a = np.sqrt(120 * 8 / np.log2(np.e)) / np.sqrt(2.0)  # LayerNorm's values there: sqrt(2)
+        q *= np.float32(a)
+        k *= np.float32(a)
+        l.w_proj *= np.float32(2.0 ** 118)
+        ids[:4] = 0, 1, 0, 1
+        ids[4:] = np.maximum(ids[4:], 2)
+    elif case == "infinite_keys":  # of tokens 0..2, in one dim of the first head
+        w.tok_emb[:, 5] = 0
+        w.tok_emb[:3, 5] = 2.0
+        w.pos_emb[:, 5] = 0
+        k[:, 7] = 0
+        k[5, 7] = np.float32(3e38)
+    ref = _one_layer_float64(w, ids)
+    m = fh.NanoLLM(w, max_batch=1)
+    try:
+        got = m.forward_window(ids[None])[0]
+    finally:
+        m.close()
+    if case == "tiny_probabilities":  # rows 0..3, 2^118 of their values, overflow in LayerNorm's variance
+        got, ref = got[4:], ref[4:]
+    nan = np.isnan(ref).any(1)
+    assert np.array_equal(np.isnan(got).any(1), nan)
+    assert (0 < nan.sum() < len(ref) - 20) if case == "infinite_keys" else not nan.any()
+    err = rel_err_rows(got[~nan], ref[~nan]).max()
+    print(f"error {err:.2e}", flush=True)
+    assert err <= 4e-6
+
+
 @pytest.mark.parametrize("name,rows", [("c4", range(1, 8)), ("c5", range(1, 4))])
 def test_large_configs_every_row_matches_oracle(name, rows):
     """Rows the fixtures do not hold (c4 rows 1-7, c5 rows 1-3): each row's prefill logits and
