@@ -147,22 +147,25 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
     const float* a_base = A + (AKC ? (size_t)row0 * lda : (size_t)row0);
     const float* b_base = B + (BKC ? (size_t)col0 * ldb : (size_t)col0);
     float va[NA][8], vb[NB][8];
+    // (not full: element e of a unit at kk is zero from kend on, read at kend - 1; loads under a
+    // condition would wait for one another)
     auto load_unit = [&](float (&v)[8], const float* base, uint32_t off, bool kc, int ld, int kk, bool full) {
         const char* p = reinterpret_cast<const char*>(base) + off;
-        if (kc) {
-            if (full) {
-                const floatx4 lo = *reinterpret_cast<const floatx4*>(p);
-                const floatx4 hi = *reinterpret_cast<const floatx4*>(p + 16);
+        if (kc && full) {
+            const floatx4 lo = *reinterpret_cast<const floatx4*>(p);
+            const floatx4 hi = *reinterpret_cast<const floatx4*>(p + 16);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
-            } else {
+            for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+        } else if (full) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = kk + e < kend ? reinterpret_cast<const float*>(p)[e] : 0.0f;
-            }
+            for (int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const float*>(p + (size_t)4 * e * ld);
         } else {
+            const ptrdiff_t step = kc ? 4 : (ptrdiff_t)4 * ld;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                v[e] = full || kk + e < kend ? *reinterpret_cast<const float*>(p + (size_t)4 * e * ld) : 0.0f;
+            for (int e = 0; e < 8; ++e) {
+                const float x = *reinterpret_cast<const float*>(p + (min(kk + e, kend - 1) - kk) * step);
+                v[e] = kk + e < kend ? x : 0.0f;
+            }
         }
     };
     auto load = [&](int k0, bool full) {
@@ -280,7 +283,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int j = 0; j < NBK; ++j) acc[i][j] += low[i][j];
+        for (int j = 0; j < NBK; ++j) acc[i][j] = (acc[i][j] + low[i][j]) * kSplitUnscale;
     if constexpr (KG == 2) {  // the second group's sums to the first
         float* sums = reinterpret_cast<float*>(all_lds);  // [register][thread]; free since the last barrier
         if (grp_k == 1) {
@@ -334,13 +337,6 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
                     for (int j = 0; j < NBK; ++j)
                         acc[i][j] = Mfma<MT>::fp32(av[i], bv[j], acc[i][j]);
             }
-        } else {
-#pragma unroll
-            for (int i = 0; i < MB; ++i)
-#pragma unroll
-                for (int j = 0; j < NBK; ++j)
-#pragma unroll
-                    for (int r = 0; r < AR; ++r) acc[i][j][r] *= kSplitUnscale;
         }
     }
 
