@@ -272,6 +272,24 @@ def test_mul_many_k_ranges(shape, mode):
     assert np.all(np.abs(dC.numpy() - A64 @ W64) <= (0.75 * K + 24) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
 
 
+@pytest.mark.parametrize("mode", [fh.NONE, fh.RIGHT])
+@pytest.mark.parametrize("shape,splits", [((70, 64, 33008), 47), ((130, 192, 16400), 24), ((66, 64, 131072), 64)])
+def test_mul_more_than_16_k_ranges(shape, splits, mode):
+    """Bound: as above, with a rounding per range; and 2-norm errors of fp32 sums of K / splits terms."""
+    M, N, K = shape
+    p = plan(M, N, K, int(mode == fh.RIGHT))
+    print(f"mul mode={mode} {shape} {p}", flush=True)
+    assert p.kind == SPLIT and p.splits == splits
+    r = _rng(M + N)
+    A, W = r.standard_normal((M, K), dtype=np.float32), r.standard_normal((K, N), dtype=np.float32)
+    dA, dW, dC = D(A), D(np.ascontiguousarray(W.T) if mode == fh.RIGHT else W), fh.DeviceArray((M, N))
+    fh.mul(mode, dC.ptr, dA.ptr, dW.ptr, M, N, K)
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    err, ref = dC.numpy() - A64 @ W64, A64 @ W64
+    assert np.all(np.abs(err) <= (0.75 * K + 8 + splits) * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64)))
+    assert np.linalg.norm(err) <= 4e-7 * np.linalg.norm(ref)
+
+
 # Row strides of 2^22 floats and more: past the split tiles' 32-bit offsets, on the fp32 tiles.
 @pytest.mark.parametrize("M,N,K,bt,lda,ldb", [(1000, 1000, 32, 0, 32, 1 << 22), (130, 4096, 32, 0, 1 << 22, 4096),
                                               (130, 4096, 32, 1, (1 << 22) + 4, 32), (4096, 130, 32, 1, 32, 1 << 22)])

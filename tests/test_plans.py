@@ -24,3 +24,15 @@ def test_row_strides_beyond_32_bit_offsets_stay_on_fp32_tiles():
         assert plan(130, 4096, 32, bt).kind == SPLIT and plan(130, 4096, 32, bt, lda=far).kind == MFMA
     assert plan(4096, 130, 32, 1, ldb=far).kind == MFMA
     assert plan(65, far, 16, 0).kind == MFMA and plan(65, 64, far, 0).kind == MFMA and plan(65, 64, far, 1).kind == MFMA
+
+
+def test_few_tiles_of_a_long_k_take_a_range_per_cu():
+    """More than 16 K ranges, while there is a CU for each; what gemm_ex plans stays within its 16 MiB."""
+    for bt in (0, 1):
+        assert plan(128, 64, 65536, bt).splits >= 48 and plan(256, 128, 65536, bt).splits == 32
+        assert plan(1024, 768, 50304, bt).splits <= 16 and plan(512, 512, 65536, bt).splits <= 16
+        for M, N in ((65, 64), (65, 384), (256, 192), (300, 300), (128, 1000)):
+            for K in (2048, 8192, 16384, 50304, 131072):
+                p, tiles = plan(M, N, K, bt), -(-M // 64) * -(-N // 64)
+                assert p.kind != SPLIT or p.splits <= 16 or (tiles * p.splits <= 256 and K >= 512 * p.splits), (M, N, K, p)
+                assert p.ws_elems <= 4 << 20
