@@ -1114,7 +1114,9 @@ namespace {
 // leave CUs idle that the wave-split kernel's 16 x 16 tiles still use (us, that kernel / this one:
 // 24 tiles 256 x 64 x 256 6.1 / 9.1, 16 tiles 256 x 256 x 2048 20 / 48; 64 tiles 512 x 64 x 512 19
 // / 14.8; 192 tiles 1024 x 64 x 1024 41 / 26; 576 tiles 3072 x 768 x 1024 96 / 49).  The error is below
-// that of that kernel's four K ranges (K 1024: 2.9e-7 / 1.9e-7).  128 x 128 tiles from two per CU on (1024 x 1024 x 64, 12 planes: 27.0 / 28.0).
+// that of that kernel's four K ranges (K 1024: 2.9e-7 / 1.9e-7).  128 x 128 tiles from two per CU on
+// (1024 x 1024 x 64, 12 planes: 27.0 / 28.0) where they compute at most a quarter more than 64 x 64
+// ones (1024 planes of 16 x 64 x 256: 51 us in large tiles, 21 in small ones; 64 x 64 x 256 47, 28).
 bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M, uint32_t N, uint32_t K, uint32_t l_rs,
                    uint32_t l_cs, uint32_t r_rs, uint32_t r_cs, uint32_t o_rs, uint32_t o_cs, uint32_t batch,
                    size_t l_plane, size_t r_plane, SplitGemm* q) {
@@ -1126,8 +1128,10 @@ bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M,
     q->A = L; q->a_kc = a_k == 1; q->lda = (int)std::min<uint32_t>(a_k == 1 ? a_r : a_k, INT32_MAX); q->a_plane = l_plane;
     q->B = R; q->b_kc = b_k == 1; q->ldb = (int)std::min<uint32_t>(b_k == 1 ? b_r : b_k, INT32_MAX); q->b_plane = r_plane;
     q->M = (int)M; q->N = (int)N; q->K = (int)K; q->planes = (int)batch;
-    q->tile = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch >= 2u * plan_cus() ? 128 : 64;
-    if (q->tile == 64) q->k_groups = split_k_groups((float)((M + 63) / 64) * ((N + 63) / 64) * batch, (int)K);
+    const uint64_t tiles = (uint64_t)((M + 63) / 64) * ((N + 63) / 64) * batch;
+    const uint64_t large = (uint64_t)((M + 127) / 128) * ((N + 127) / 128) * batch;
+    q->tile = large >= 2u * plan_cus() && 16 * large <= 5 * tiles ? 128 : 64;
+    if (q->tile == 64) q->k_groups = split_k_groups((float)tiles, (int)K);
     return gemm_split_takes(*q);
 }
 }  // namespace

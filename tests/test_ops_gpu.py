@@ -353,6 +353,24 @@ def test_matmul_strided_split_tiles(shape, swap, mode):
     assert np.all(got[:, :, N:] == 7.0)
 
 
+# Many small planes: 64 x 64 tiles, however many there are.
+@pytest.mark.parametrize("mode", [fh.NONE, fh.RIGHT, fh.LEFT])
+@pytest.mark.parametrize("M,N,K", [(16, 64, 256), (64, 28, 16), (24, 72, 64), (48, 64, 64)])
+def test_matmul_strided_many_small_planes(M, N, K, mode):
+    planes = 600
+    r = _rng(M + K)
+    A = r.standard_normal((planes, M, K), dtype=np.float32)
+    B = r.standard_normal((planes, K, N), dtype=np.float32)
+    L = np.ascontiguousarray(np.swapaxes(A, 1, 2) if mode == fh.LEFT else A)
+    R = np.ascontiguousarray(np.swapaxes(B, 1, 2) if mode == fh.RIGHT else B)
+    dL, dR, dO = D(L), D(R), fh.DeviceArray((planes, M, N))
+    args = (mode, M, N, K, L.shape[2], 1, R.shape[2], 1, N, 1, planes, M * K, K * N)
+    assert strided_tile(*args) == 64
+    fh.matmul_strided(mode, dO.ptr, dL.ptr, dR.ptr, *args[1:], M * N)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(dO.numpy() - A64 @ B64) <= (0.75 * K + 8) * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)))
+
+
 @pytest.mark.parametrize("epi", [fh.EPI_GELU, fh.EPI_RESID])
 @pytest.mark.parametrize("tile", ["128x128", "64x64"])
 def test_gemm_nt_kernel_epilogues_in_place(epi, tile, monkeypatch):

@@ -1,7 +1,8 @@
 """Plans of the products, on the host (256 CUs where there is no device)."""
 import random
 
-from plans import MFMA, SPLIT, engine_workspace, plan
+import freeml_amd as fh
+from plans import MFMA, SPLIT, engine_workspace, plan, strided_tile
 
 
 def test_engine_workspace_holds_every_product_of_a_prefill():
@@ -36,3 +37,17 @@ def test_few_tiles_of_a_long_k_take_a_range_per_cu():
                 p, tiles = plan(M, N, K, bt), -(-M // 64) * -(-N // 64)
                 assert p.kind != SPLIT or p.splits <= 16 or (tiles * p.splits <= 256 and K >= 512 * p.splits), (M, N, K, p)
                 assert p.ws_elems <= 4 << 20
+
+
+def _packed_planes(mode, M, N, K, planes):
+    l = {fh.NONE: K, fh.RIGHT: K, fh.LEFT: M}[mode], 1
+    r = {fh.NONE: N, fh.RIGHT: K, fh.LEFT: N}[mode], 1
+    return strided_tile(mode, M, N, K, *l, *r, N, 1, planes, M * K, N * K)
+
+
+def test_large_strided_tiles_only_where_they_are_filled():
+    for mode in (fh.NONE, fh.RIGHT, fh.LEFT):
+        for M, N in ((64, 64), (16, 64), (24, 256), (100, 48), (192, 64), (130, 120)):
+            assert _packed_planes(mode, M, N, 64, 2048) == 64, (M, N)
+        assert _packed_planes(mode, 1024, 1024, 64, 12) == 128 and _packed_planes(mode, 128, 128, 64, 1024) == 128
+        assert _packed_planes(mode, 120, 252, 64, 1024) == 128 and _packed_planes(mode, 1024, 64, 1024, 12) == 64
