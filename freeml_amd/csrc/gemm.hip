@@ -1122,6 +1122,9 @@ bool strided_split(bool tl, bool tr, const float* L, const float* R, uint32_t M,
                    size_t l_plane, size_t r_plane, SplitGemm* q) {
     if (o_cs != 1 || o_rs > INT32_MAX || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || batch > 65535) return false;
     if ((double)M * N * batch < 64.0 * 64 * 64) return false;
+    // Planes of a quarter tile beyond one per CU stay on that kernel's 32 x 32 tiles but for the shortest
+    // K (32 x 32 x 256: 256 planes 10 / 8.5 us, 400 10 / 12, 1024 x 32 x 32 x 64 7.1 / 9.5, 600 x 32 x 32 x 16 6 / 5.5).
+    if (M <= 32 && N <= 32 && K > 32 && batch > (uint32_t)plan_cus()) return false;
     // Strides between the k of one row of A (column of B) and between its rows (columns).
     const uint32_t a_k = tl ? l_rs : l_cs, a_r = tl ? l_cs : l_rs, b_k = tr ? r_cs : r_rs, b_r = tr ? r_rs : r_cs;
     if ((a_k != 1 && a_r != 1) || (b_k != 1 && b_r != 1)) return false;

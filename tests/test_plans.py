@@ -51,3 +51,10 @@ def test_large_strided_tiles_only_where_they_are_filled():
             assert _packed_planes(mode, M, N, 64, 2048) == 64, (M, N)
         assert _packed_planes(mode, 1024, 1024, 64, 12) == 128 and _packed_planes(mode, 128, 128, 64, 1024) == 128
         assert _packed_planes(mode, 120, 252, 64, 1024) == 128 and _packed_planes(mode, 1024, 64, 1024, 12) == 64
+
+
+def test_planes_of_a_quarter_tile_stay_on_the_vector_kernel():
+    for mode in (fh.NONE, fh.RIGHT, fh.LEFT):
+        assert _packed_planes(mode, 32, 32, 64, 1024) == 0 and _packed_planes(mode, 16, 20, 256, 2048) == 0
+        assert _packed_planes(mode, 32, 32, 256, 256) == 64 and _packed_planes(mode, 32, 32, 32, 1024) == 64
+        assert _packed_planes(mode, 36, 32, 64, 1024) == 64
