@@ -29,9 +29,6 @@
 #include "bf16_split.h"
 #include "gemm_split.h"
 
-#include <cstdlib>
-#include <cstring>
-
 namespace fmlh {
 
 namespace {
@@ -404,11 +401,8 @@ int launch(const SplitGemm& g) {
     const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
     constexpr size_t lds = (size_t)KG * 2 * 3 * (BM + BN) * BK * sizeof(uint16_t);  // 48 KB per group
     auto kern = gemm_split_kernel<BM, BN, BK, 2, 2, KG, AKC, BKC, EPI, SPLIT, BM == 128 ? 32 : 16>;
-    if constexpr (lds > 64 * 1024) {
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        FMLH_HIP(attr);
-    }
+    if constexpr (lds > 64 * 1024)  // each time: the library may have been started on another device since
+        FMLH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)tm * tn, 1, SPLIT ? g.splits : g.planes), dim3(256 * KG), lds, g.s, g.A, g.lda,
                        g.a_plane, g.B, g.ldb, g.b_plane, g.C, g.ldc, g.c_plane, g.M, g.N, g.K, g.R, g.ldr, g.kv,
                        g.partial, g.k_per_split, tm, tn);
