@@ -148,11 +148,15 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
     // condition would wait for one another)
     auto load_unit = [&](float (&v)[8], const float* base, uint32_t off, bool kc, int ld, int kk, bool full) {
         const char* p = reinterpret_cast<const char*>(base) + off;
-        if (kc && full) {
-            const floatx4 lo = *reinterpret_cast<const floatx4*>(p);
-            const floatx4 hi = *reinterpret_cast<const floatx4*>(p + 16);
+        if (kc && (full || kend % 8 == 0)) {  // units are whole or past the end
+            const char* q = full ? p : p + 4 * (min(kk, kend - 8) - kk);
+            const floatx4 lo = *reinterpret_cast<const floatx4*>(q);
+            const floatx4 hi = *reinterpret_cast<const floatx4*>(q + 16);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+            for (int e = 0; e < 4; ++e) {
+                v[e] = full || kk < kend ? lo[e] : 0.0f;
+                v[4 + e] = full || kk < kend ? hi[e] : 0.0f;
+            }
         } else if (full) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const float*>(p + (size_t)4 * e * ld);
