@@ -1037,10 +1037,16 @@ int gemm(const GemmArgs& g, float* ws, size_t ws_elems) {
         return gemm_strided(g.b_trans ? FMLH_TRANSPOSE_RIGHT : FMLH_TRANSPOSE_NONE, g.C, g.A, g.B,
                             g.M, g.N, g.K, g.lda, 1, g.ldb, 1, g.ldc, 1, 1, 0, 0, 0, g.s);
     }
-    const GemmPlan p = plan_for(g);
+    GemmPlan p = plan_for(g);
     if (p.ws_elems > ws_elems) {
         if (ws != nullptr) return set_error(FMLH_E_INVALID, "gemm: workspace too small");
-        FMLH_TRY(global_workspace(p.ws_elems, &ws));
+        const int rc = global_workspace(p.ws_elems, &ws);
+        if (rc != FMLH_OK && p.kind != GemmPlan::kSplit) return rc;
+        if (rc != FMLH_OK) {  // no room for partials: one K range
+            (void)hipGetLastError();
+            clear_error();
+            p.splits = 1;
+        }
     }
     switch (p.kind) {
         case GemmPlan::kSkinnyNT:

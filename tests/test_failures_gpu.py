@@ -141,3 +141,33 @@ def test_every_forced_failure_surfaces_and_leaves_nothing_stale(kind, path):
 
 def test_shutdown_releases_engines_and_refuses_stale_handles():
     assert "SHUTDOWN_OK" in _run(SHUTDOWN)
+
+
+NO_ROOM = r"""
+import os, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+import freeml_amd as fh
+
+fh.init(0)
+r = np.random.default_rng(1)
+A, W = r.standard_normal((500, 4096), dtype=np.float32), r.standard_normal((4096, 384), dtype=np.float32)
+D = fh.DeviceArray.from_host
+dA, dW, dT, dC = D(A), D(W), D(np.ascontiguousarray(W.T)), fh.DeviceArray((500, 384))
+ref = A.astype(np.float64) @ W
+for mode, w in ((fh.NONE, dW), (fh.RIGHT, dT)):
+    os.environ["FMLH_FAULT"] = "alloc:1"
+    fh.init(0)  # re-arms the hook: the next allocation fails
+    fh.mul(mode, dC.ptr, dA.ptr, w.ptr, 500, 384, 4096)
+    assert np.abs(dC.numpy() - ref).max() <= 1e-5 * np.abs(ref).max(), mode
+    print("no room for partials: mode", mode, flush=True)
+os.environ.pop("FMLH_FAULT")
+fh.init(0)
+fh.mul(fh.NONE, dC.ptr, dA.ptr, dW.ptr, 500, 384, 4096)  # in K ranges
+assert np.abs(dC.numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+"""
+
+
+def test_products_without_room_for_partials_take_one_k_range():
+    r = subprocess.run([sys.executable, "-u", "-c", NO_ROOM.format(root=ROOT)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
