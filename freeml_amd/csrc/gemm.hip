@@ -3,8 +3,8 @@
 //  * gemm_split_kernel (gemm_split.hip): everything wider than the batched decode, each fp32
 //    operand split into three bf16 parts on the bf16 matrix cores.
 //  * gemm_mfma_kernel: fp32 MFMA tiles (v_mfma_f32_32x32x2f32) with register-staged,
-//    double-buffered LDS, for either B layout and 8 < M <= 64 (batched decode).  Optional
-//    split-K writes partial sums that splitk_reduce_kernel adds in a fixed order
+//    double-buffered LDS, for either B layout: 8 < M <= 64 (batched decode), the smallest
+//    products above, and row strides past the split tiles' 32-bit offsets.  Optional split-K writes partial sums that splitk_reduce_kernel adds in a fixed order
 //    (deterministic) before the epilogue.
 //  * skinny kernels for M <= 8 (single-sequence decode): HBM-bound weight streaming, every
 //    weight read once, all M rows accumulated per weight load.
@@ -914,8 +914,8 @@ GemmPlan plan_gemm(int M, int N, int K, int b_trans, bool one_range, size_t ws_m
     if (split_takes && ((M > 64 && !small) || (b_trans && 2 * tiles64 >= cus))) {
         p.kind = GemmPlan::kSplit;
         // Tile and K ranges by the time (us) they take, fitted on MI355X to 266 shapes (256 .. 14336
-        // rows of 384 .. 1024-wide blocks, K to 50304) x 2 layouts x up to 15 choices: 0.5 % behind the
-        // best choice on average, 11 % at worst.  A CU multiplies a 128 x 128 x 16 block in 0.62 us
+        // rows of 384 .. 1024-wide blocks, K to 50304) x 2 layouts x up to 15 choices: 1 % behind the
+        // best choice on average, 12 % at worst.  A CU multiplies a 128 x 128 x 16 block in 0.62 us
         // whether it holds one work-group or two, a 64 x 64 x 32 one in 0.64 alone (0.70 with B stored
         // K x N), 0.45 (0.50) by two groups of waves that share the K range, and 0.41 among several
         // work-groups; K ranges write and read their partials, and the reduction is a launch.  What

@@ -1,7 +1,9 @@
 // fp32 products on the bf16 matrix cores: gemm_split_kernel.
 //
 // Every fp32 operand element is split exactly into three bf16 parts, x = x0 + x1 + x2 (each the
-// round-to-nearest bf16 of what is left, 3 x 8 significant bits = fp32's 24), and the product
+// round-to-nearest bf16 of what is left, 3 x 8 significant bits = fp32's 24; the method of Henry, Tang
+// and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019), and the product
 // takes the six part products whose weight is 2^-16 or more of the whole,
 //   a b ~ a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0),
 // accumulated in fp32 by the bf16 MFMAs: a0 b0 in one accumulator, the five small ones, smallest
@@ -21,9 +23,10 @@
 //
 // The operands are split while they are staged (registers -> LDS), so fp32 matrices of any
 // layout are read once and nothing is kept.  Per 128 x 128 x 16 block a work-group's matrix cores
-// need ~770 clocks, its LDS ~580 (three planes written once, read by two waves) and its
-// vector units ~540 (6 instructions per element); 64 x 64 tiles are bound by LDS (two waves read
-// every plane of half as many products) and serve the products with too few large tiles.  The
+// need 768 clocks, its LDS 580 (three planes written once, read by two waves; 192 of them bank
+// conflicts) and its vector units 600 (6 instructions per element and the addresses); per 64 x 64 x 32
+// block, with half as many products per element, 384, 390 and 640 (counters).  The small tiles serve
+// the products with too few large ones.  The
 // launch bounds matter: left alone, the compiler takes 267 registers for the large tile (one wave
 // per SIMD: 4096 x 3072 x 768 125 us instead of 107).
 #include "bf16_split.h"

@@ -282,9 +282,9 @@ def test_persistent_decode_matches_multikernel_path(name, batch):
                                                ("c2", 129, 2), ("c2", 64, 3), ("c5", 700, 1),
                                                ("c5", 1920, 2)])
 def test_prefill_attention_on_matrix_cores_matches_per_lane_kernel(kernel, name, length, batch):
-    """The MFMA prefill attention kernels for head_dim 64 (default: 32x32x2 MFMA with 128
-    queries per work-group from 256 rows on, else 16x16x4 with 64; FMLH_ATTN_PREFILL=mfma16 /
-    mfma32: one of them at every length) and the per-lane kernel
+    """The MFMA prefill attention kernels for head_dim 64 (default: three bf16 parts with
+    128 queries per work-group from 256 rows on, else 16x16x4 fp32 with 64; FMLH_ATTN_PREFILL=
+    mfma16 / mfma32: the latter / the former at every length) and the per-lane kernel
     (FMLH_ATTN_PREFILL=simt) give the same prefill logits (every sequence's last row) to fp32
     reassociation, for full and partial query blocks, one key tile, and several sequences."""
     print(f"prefill attention {kernel} {name} length {length} batch {batch}", flush=True)
@@ -1084,8 +1084,8 @@ def test_wide_epoch_count_wraps_cleanly():
 @pytest.mark.parametrize("C,H,B,P,parts", [(1024, 16, 16, 64, "2"), (1024, 16, 1, 576, "2"),
                                            (384, 6, 22, 64, "4")])
 def test_fused_prefill_part_workspace(C, H, B, P, parts):
-    """Each part of the fused prefill gets a workspace slice sized for what its QKV and FC
-    products plan at the part's rows (they can split K where a part is small) -- C = 1024 at
+    """Each part of the fused prefill gets a workspace slice sized for its rows and the K ranges its
+    products plan for the rows of all parts -- C = 1024 at
     16 x 64 and 1 x 576 rows, and four parts of c3's width at 22 sequences.  Every sequence's
     prefill logits and first decode step against the oracle, on a one-layer model."""
     shape = synth.NanoLLMShape(65, 640, C, H, 1)
