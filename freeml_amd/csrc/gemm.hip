@@ -4,8 +4,9 @@
 //    operand split into three bf16 parts on the bf16 matrix cores.
 //  * gemm_mfma_kernel: fp32 MFMA tiles (v_mfma_f32_32x32x2f32) with register-staged,
 //    double-buffered LDS, for either B layout: 8 < M <= 64 (batched decode), the smallest
-//    products above, and row strides past the split tiles' 32-bit offsets.  Optional split-K writes partial sums that splitk_reduce_kernel adds in a fixed order
-//    (deterministic) before the epilogue.
+//    products above, and row strides past the split tiles' 32-bit offsets.  Optional split-K
+//    writes partial sums that splitk_reduce_kernel adds in a fixed order (deterministic) before
+//    the epilogue.
 //  * skinny kernels for M <= 8 (single-sequence decode): HBM-bound weight streaming, every
 //    weight read once, all M rows accumulated per weight load.
 //  * gemm_strided_kernel: any transpose mode and element strides (MatMul_Strided views).
