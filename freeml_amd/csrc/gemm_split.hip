@@ -259,23 +259,45 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
     const int nk = max(kend - kbeg, 0) / BK;
     const int nk_all = KG == 1 ? nk : (min(kend_wg, kbeg_wg + k_half) - kbeg_wg) / BK;
     const bool rest = kbeg + nk * BK < kend;
-    if (nk_all > 0) {
+    if constexpr (KG == 1) {
         if (nk > 0) {
             load(kbeg, true);
             store(0);
-            load(kbeg + (nk > 1 ? BK : 0), true);
+            if (nk > 1) load(kbeg + BK, true);
         }
         barrier();
-        for (int kb = 0; kb < nk_all; ++kb) {
-            if (KG == 1 || kb < nk)
-                multiply(kb & 1, [&]() {
-                    store((kb + 1) & 1);
-                    load(kbeg + min(kb + 2, nk - 1) * BK, true);
-                });
+        for (int kb = 0; kb + 1 < nk; ++kb) {
+            multiply(kb & 1, [&]() {
+                store((kb + 1) & 1);
+                load(kbeg + min(kb + 2, nk - 1) * BK, true);
+            });
             barrier();
         }
-    }
-    if (KG == 2 || rest) {  // the rest of K
+        if (rest) load(kbeg + nk * BK, false);
+        if (nk > 0) multiply((nk - 1) & 1, []() {});
+        if (rest) {
+            store(nk & 1);
+            barrier();
+            multiply(nk & 1, []() {});
+        }
+        barrier();
+    } else {
+        if (nk_all > 0) {
+            if (nk > 0) {
+                load(kbeg, true);
+                store(0);
+                load(kbeg + (nk > 1 ? BK : 0), true);
+            }
+            barrier();
+            for (int kb = 0; kb < nk_all; ++kb) {
+                if (kb < nk)
+                    multiply(kb & 1, [&]() {
+                        store((kb + 1) & 1);
+                        load(kbeg + min(kb + 2, nk - 1) * BK, true);
+                    });
+                barrier();
+            }
+        }
         if (rest) {
             load(kbeg + nk * BK, false);
             store(0);
