@@ -334,14 +334,14 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG, KG == 2 || BM == 128 ? 2 : 3) 
     // What leaves the range is multiplied again in fp32: infinities and elements that scaled or rounded
     // to bf16 become one, which leave a NaN in the sums, and sums past the scaled range.
     {
-        bool redo = false;
+        float bad = 0.0f;  // zero as long as every sum is finite (an or of comparisons: 9.8 -> 10.3 us at 9000 x 384 x 64)
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
             for (int j = 0; j < NBK; ++j)
 #pragma unroll
-                for (int r = 0; r < AR; ++r) redo |= !(fabsf(acc[i][j][r]) < INFINITY);
-        if (__syncthreads_or(redo)) {
+                for (int r = 0; r < AR; ++r) bad = fmaf(acc[i][j][r], 0.0f, bad);
+        if (__syncthreads_or(bad != 0.0f)) {
             clear();
             for (int k = kbeg_wg; k < kend_wg; k += 64 / MT) {
                 const int kk = min(k + h, kend_wg - 1);
